@@ -336,6 +336,14 @@ int shx_norm_pow(const float* x, int64_t n, double p, double* out, void* stream)
 int shx_band_mad(const float* planes, long long plane_elems, long long plane_stride, int nplanes, int arith,
                  double* mad, void* stream);
 
+/* shx_band_mad with a device workspace of at least
+ * shx_band_mad_workspace(plane_elems, nplanes) bytes (16-byte aligned; NULL
+ * or 0 bytes where that is 0), over which planes of more than 32768 elements
+ * are split over many workgroups instead of one each.  Same results. */
+size_t shx_band_mad_workspace(long long plane_elems, int nplanes);
+int shx_band_mad_ws(const float* planes, long long plane_elems, long long plane_stride, int nplanes, int arith,
+                    double* mad, void* work, size_t work_bytes, void* stream);
+
 /* Noise scalars of a dictionary: the transform of the given noise image
  * (L x L device FP32, normally unit white noise), then shx_band_mad of every
  * band, into scalars[0 .. nbands] on the host (lowpass first, then the bands

@@ -90,6 +90,9 @@ _SIGNATURES = [
     ("shx_norm_pow", c_int, [c_void_p, c_int64, c_double, P(c_double), c_void_p]),
     ("shx_softth", c_int, [c_void_p, c_int64, c_double, c_void_p]),
     ("shx_band_mad", c_int, [c_void_p, ctypes.c_longlong, ctypes.c_longlong, c_int, c_int, c_void_p, c_void_p]),
+    ("shx_band_mad_workspace", c_size_t, [ctypes.c_longlong, c_int]),
+    ("shx_band_mad_ws", c_int, [c_void_p, ctypes.c_longlong, ctypes.c_longlong, c_int, c_int, c_void_p, c_void_p,
+                                c_size_t, c_void_p]),
     ("shx_nsst_scalars", c_int, [c_void_p, c_void_p, c_int, P(c_double), c_void_p]),
     ("shx_separate", c_int, [c_void_p, c_void_p, c_int, c_int, c_double, c_double, P(c_double), c_int, P(c_double),
                              c_int, c_double, P(c_double), c_int, c_int, c_void_p, c_void_p, P(c_double), c_void_p]),

@@ -521,8 +521,10 @@ def band_mad_cuda(planes, arith="fp64"):
     pe = planes.numel() // max(n, 1)
     out = torch.empty(n, device=planes.device, dtype=torch.float64)
     if n:
-        check(lib.shx_band_mad(ctypes.c_void_p(planes.data_ptr()), pe, pe, n, MAD_ARITH[arith],
-                               ctypes.c_void_p(out.data_ptr()), _stream()))
+        nbytes = int(lib.shx_band_mad_workspace(pe, n))
+        work = _workspace(nbytes // 4, planes.device) if nbytes else None
+        check(lib.shx_band_mad_ws(ctypes.c_void_p(planes.data_ptr()), pe, pe, n, MAD_ARITH[arith],
+                                  ctypes.c_void_p(out.data_ptr()), _vp(work) if nbytes else None, nbytes, _stream()))
     return out
 
 

@@ -1572,9 +1572,10 @@ int shx_nsst_scalars(shx_dict* d, const float* noise, int arith, double* scalars
   if (arith != SHX_MAD_FP64 && arith != SHX_MAD_FP32) return fail(SHX_ERR_ARG, "unknown arithmetic %d", arith);
   const size_t pl = d->plane(), np = 1 + (size_t)d->nbands;
   hipStream_t s = (hipStream_t)stream;
-  float* stack = nullptr;
+  float* stack = nullptr;  // the coefficients, then the workspace of the medians
   double* mad = nullptr;
-  hipError_t e = hipMalloc(&stack, sizeof(float) * pl * np);
+  const size_t wb = shx_band_mad_workspace((long long)pl, (int)np);
+  hipError_t e = hipMalloc(&stack, sizeof(float) * pl * np + wb);
   if (e == hipSuccess) e = hipMalloc(&mad, sizeof(double) * np);
   if (e != hipSuccess) {
     if (stack) (void)hipFree(stack);
@@ -1586,7 +1587,8 @@ int shx_nsst_scalars(shx_dict* d, const float* noise, int arith, double* scalars
   std::vector<Stage> st;
   stages_dec(d, d->w, 1, noise, 0, cell_coeffs(d, cells.data()), s, st);
   int r = run_stages(st);
-  if (r == SHX_OK) r = shx_band_mad(stack, (long long)pl, (long long)pl, (int)np, arith, mad, stream);
+  if (r == SHX_OK)
+    r = shx_band_mad_ws(stack, (long long)pl, (long long)pl, (int)np, arith, mad, stack + pl * np, wb, stream);
   if (r == SHX_OK && ((e = hipMemcpyAsync(scalars, mad, sizeof(double) * np, hipMemcpyDeviceToHost, s)) != hipSuccess ||
                       (e = hipStreamSynchronize(s)) != hipSuccess))
     r = fail(SHX_ERR_HIP, "scalar download failed: %s", hipGetErrorString(e));
@@ -2498,7 +2500,11 @@ extern "C" int shx_separate(shx_dict* d, const float* img, int level2, int iterm
       if (!ok(shx_mrdwt(x, L, L, d4.data(), 4, 1, t, yh, work, 1, stream))) break;   // separate.m:81-101
       hipLaunchKernelGGL(k_even_hh, dim3((unsigned)std::min<size_t>(1024, (pl / 4 + 255) / 256)), dim3(256), 0, s,
                          yh, L, hh);
-      if (!ok(shx_band_mad(hh, (long long)(pl / 4), (long long)(pl / 4), 1, SHX_MAD_FP64, dmad, stream))) break;
+      // the coefficient stack is free here: workspace of the median (1 + nb
+      // planes; a plane that needs one has at least 4 * 32768 elements)
+      if (!ok(shx_band_mad_ws(hh, (long long)(pl / 4), (long long)(pl / 4), 1, SHX_MAD_FP64, dmad, stack,
+                              sizeof(float) * (1 + (size_t)nb) * pl, stream)))
+        break;
       if (hipMemcpyAsync(&sigma, dmad, sizeof(double), hipMemcpyDeviceToHost, s) != hipSuccess ||
           hipStreamSynchronize(s) != hipSuccess) {
         rc = fail(SHX_ERR_HIP, "noise level download failed");

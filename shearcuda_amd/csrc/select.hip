@@ -57,71 +57,120 @@ struct KeyDev32 {
   __device__ uint64_t operator()(float v) const { return __float_as_uint(fabsf(v - m)); }
 };
 
-template <bool VEC, class K, class F>
-__device__ __forceinline__ void each_key(const float* __restrict__ p, int n, const K& kf, F&& fn) {
+// Calls fn(v) for every element of p[0, n) over the block's NT threads.
+template <bool VEC, int NT, class F>
+__device__ __forceinline__ void each_value(const float* __restrict__ p, int n, F&& fn) {
   int i0 = 0;
   if constexpr (VEC) {
     const float4* p4 = reinterpret_cast<const float4*>(p);
     const int n4 = n >> 2;
-    for (int i = threadIdx.x; i < n4; i += MT) {
+    int i = threadIdx.x;
+    // four loads in flight: fn's LDS atomics keep the compiler from moving
+    // the next load above them
+    for (; i + 3 * NT < n4; i += 4 * NT) {
+      float4 v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = p4[i + u * NT];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        fn(v[u].x);
+        fn(v[u].y);
+        fn(v[u].z);
+        fn(v[u].w);
+      }
+    }
+    for (; i < n4; i += NT) {
       const float4 v = p4[i];
-      fn(kf(v.x));
-      fn(kf(v.y));
-      fn(kf(v.z));
-      fn(kf(v.w));
+      fn(v.x);
+      fn(v.y);
+      fn(v.z);
+      fn(v.w);
     }
     i0 = n4 << 2;
   }
-  for (int i = i0 + threadIdx.x; i < n; i += MT) fn(kf(p[i]));
+  for (int i = i0 + threadIdx.x; i < n; i += NT) fn(p[i]);
 }
 
 struct SelShared {
   uint32_t hist[MBINS];
   uint32_t wsum[MT / 64];
   uint32_t res[3];
-  uint64_t wmin[MT / 64];
+  uint64_t wmin[MT / 64], wmax[MT / 64];
 };
 
-// Key of the element of rank k (0-based) of the plane under kf; *after_eq is
-// the number of elements with the same key ranked after it.
-template <bool VEC, class K>
-__device__ uint64_t block_select(const float* __restrict__ p, int n, uint32_t k, const K& kf, SelShared& sh,
-                                 uint32_t* after_eq) {
+// Rank search in a histogram held by `sh`, two bins per thread: the bin that
+// holds rank krem, the elements before it and in it go to sh.res.
+__device__ __forceinline__ void find_bin(SelShared& sh, uint32_t krem) {
   const int t = threadIdx.x;
-  uint64_t prefix = 0, pmask = 0;
-  uint32_t krem = k, cnt = 0;
-  for (int left = K::W; left > 0;) {
+  const uint32_t h0 = sh.hist[2 * t], h1 = sh.hist[2 * t + 1], s = h0 + h1;
+  uint32_t inc = s;
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t y = __shfl_up(inc, o, 64);
+    if ((t & 63) >= o) inc += y;
+  }
+  if ((t & 63) == 63) sh.wsum[t >> 6] = inc;
+  __syncthreads();
+  uint32_t before = inc - s;
+  for (int w = 0; w < (t >> 6); ++w) before += sh.wsum[w];
+  if (krem >= before && krem < before + h0) {
+    sh.res[0] = 2 * t;
+    sh.res[1] = before;
+    sh.res[2] = h0;
+  } else if (krem >= before + h0 && krem < before + s) {
+    sh.res[0] = 2 * t + 1;
+    sh.res[1] = before + h0;
+    sh.res[2] = h1;
+  }
+  __syncthreads();
+}
+
+__device__ __forceinline__ uint64_t shfl_xor64(uint64_t v, int o) {
+  const uint32_t lo = __shfl_xor((uint32_t)v, o, 64), hi = __shfl_xor((uint32_t)(v >> 32), o, 64);
+  return ((uint64_t)hi << 32) | lo;
+}
+
+// Smallest and largest of the block's values.
+__device__ __forceinline__ void block_minmax(uint64_t& mn, uint64_t& mx, SelShared& sh) {
+  const int t = threadIdx.x;
+  for (int o = 32; o > 0; o >>= 1) {
+    const uint64_t a = shfl_xor64(mn, o), b = shfl_xor64(mx, o);
+    mn = a < mn ? a : mn;
+    mx = b > mx ? b : mx;
+  }
+  if ((t & 63) == 0) sh.wmin[t >> 6] = mn, sh.wmax[t >> 6] = mx;
+  __syncthreads();
+  mn = sh.wmin[0], mx = sh.wmax[0];
+  for (int w = 1; w < MT / 64; ++w) {
+    mn = sh.wmin[w] < mn ? sh.wmin[w] : mn;
+    mx = sh.wmax[w] > mx ? sh.wmax[w] : mx;
+  }
+  __syncthreads();
+}
+
+// Key of the element of rank k (0-based) of p[0, n) under kf; *after_eq is
+// the number of elements with the same key ranked after it.  All keys lie in
+// [kmin, kmax], so the passes start at the highest bit in which these differ.
+template <bool VEC, class K>
+__device__ uint64_t block_select(const float* __restrict__ p, int n, uint32_t k, const K& kf, uint64_t kmin,
+                                 uint64_t kmax, SelShared& sh, uint32_t* after_eq) {
+  const int t = threadIdx.x;
+  const int top = kmin == kmax ? 0 : 64 - __clzll((long long)(kmin ^ kmax));
+  uint64_t pmask = top == 64 ? 0 : ~0ull << top;
+  uint64_t prefix = kmin & pmask;
+  uint32_t krem = k, cnt = (uint32_t)n;
+  for (int left = top; left > 0;) {
     const int d = left < MBITS ? left : MBITS;
     const int shift = left - d;
     const uint32_t dmask = (1u << d) - 1u;
     sh.hist[2 * t] = 0;
     sh.hist[2 * t + 1] = 0;
     __syncthreads();
-    each_key<VEC>(p, n, kf, [&](uint64_t key) {
+    each_value<VEC, MT>(p, n, [&](float v) {
+      const uint64_t key = kf(v);
       if ((key & pmask) == prefix) atomicAdd(&sh.hist[(uint32_t)(key >> shift) & dmask], 1u);
     });
     __syncthreads();
-    // exclusive scan over the bins: thread t owns bins 2t and 2t+1
-    const uint32_t h0 = sh.hist[2 * t], h1 = sh.hist[2 * t + 1], s = h0 + h1;
-    uint32_t inc = s;
-    for (int o = 1; o < 64; o <<= 1) {
-      const uint32_t y = __shfl_up(inc, o, 64);
-      if ((t & 63) >= o) inc += y;
-    }
-    if ((t & 63) == 63) sh.wsum[t >> 6] = inc;
-    __syncthreads();
-    uint32_t before = inc - s;
-    for (int w = 0; w < (t >> 6); ++w) before += sh.wsum[w];
-    if (krem >= before && krem < before + h0) {
-      sh.res[0] = 2 * t;
-      sh.res[1] = before;
-      sh.res[2] = h0;
-    } else if (krem >= before + h0 && krem < before + s) {
-      sh.res[0] = 2 * t + 1;
-      sh.res[1] = before + h0;
-      sh.res[2] = h1;
-    }
-    __syncthreads();
+    find_bin(sh, krem);
     krem -= sh.res[1];
     cnt = sh.res[2];
     prefix |= (uint64_t)sh.res[0] << shift;
@@ -133,70 +182,371 @@ __device__ uint64_t block_select(const float* __restrict__ p, int n, uint32_t k,
   return prefix;
 }
 
-// Smallest key above `above` (exists whenever the caller asks for it).
+// The keys of ranks k and k + 1 (the latter only if `two`) of p[0, n); `above`
+// is the smallest key past the array (the answer if rank k is its last).
 template <bool VEC, class K>
-__device__ uint64_t block_min_above(const float* __restrict__ p, int n, uint64_t above, const K& kf, SelShared& sh) {
-  const int t = threadIdx.x;
-  uint64_t mn = ~0ull;
-  each_key<VEC>(p, n, kf, [&](uint64_t key) {
-    if (key > above && key < mn) mn = key;
+__device__ void block_pair(const float* __restrict__ p, int n, uint32_t k, bool two, uint64_t above, const K& kf,
+                           uint64_t kmin, uint64_t kmax, SelShared& sh, uint64_t* lo, uint64_t* hi) {
+  uint32_t after = 0;
+  *lo = *hi = block_select<VEC>(p, n, k, kf, kmin, kmax, sh, &after);
+  if (!two || after > 0) return;
+  uint64_t mn = above, mx = 0;
+  each_value<VEC, MT>(p, n, [&](float v) {
+    const uint64_t key = kf(v);
+    if (key > *lo && key < mn) mn = key;
   });
-  for (int o = 32; o > 0; o >>= 1) {
-    const uint32_t lo = __shfl_xor((uint32_t)mn, o, 64), hi = __shfl_xor((uint32_t)(mn >> 32), o, 64);
-    const uint64_t y = ((uint64_t)hi << 32) | lo;
-    mn = y < mn ? y : mn;
-  }
-  if ((t & 63) == 0) sh.wmin[t >> 6] = mn;
-  __syncthreads();
-  uint64_t r = sh.wmin[0];
-  for (int w = 1; w < MT / 64; ++w) r = sh.wmin[w] < r ? sh.wmin[w] : r;
-  __syncthreads();
-  return r;
+  block_minmax(mn, mx, sh);
+  *hi = mn;
 }
 
-// The two middle keys (equal for an odd count).
+// The two middle keys of a whole plane (equal for an odd count).
 template <bool VEC, class K>
 __device__ void block_middle(const float* __restrict__ p, int n, const K& kf, SelShared& sh, uint64_t* lo,
                              uint64_t* hi) {
-  uint32_t after = 0;
-  if (n & 1) {
-    *lo = *hi = block_select<VEC>(p, n, (uint32_t)(n / 2), kf, sh, &after);
-    return;
-  }
-  *lo = block_select<VEC>(p, n, (uint32_t)(n / 2 - 1), kf, sh, &after);
-  *hi = after > 0 ? *lo : block_min_above<VEC>(p, n, *lo, kf, sh);
+  uint64_t mn = ~0ull, mx = 0;
+  each_value<VEC, MT>(p, n, [&](float v) {
+    const uint64_t key = kf(v);
+    mn = key < mn ? key : mn;
+    mx = key > mx ? key : mx;
+  });
+  block_minmax(mn, mx, sh);
+  block_pair<VEC>(p, n, (uint32_t)((n - 1) / 2), !(n & 1), ~0ull, kf, mn, mx, sh, lo, hi);
 }
 
-template <bool VEC, bool FP32>
+// Median of the values from its two middle keys.
+template <bool FP32>
+__device__ __forceinline__ double value_median(uint64_t a, uint64_t b, int n) {
+  const float fa = f32_unkey((uint32_t)a), fb = f32_unkey((uint32_t)b);
+  if constexpr (FP32) return (n & 1) ? fa : (fa + fb) / 2.0f;
+  return (n & 1) ? (double)fa : ((double)fa + (double)fb) / 2.0;
+}
+// MAD / 0.6745 from the two middle deviation keys.
+template <bool FP32>
+__device__ __forceinline__ double dev_mad(uint64_t a, uint64_t b, int n) {
+  if constexpr (FP32) {
+    const float da = __uint_as_float((uint32_t)a), db = __uint_as_float((uint32_t)b);
+    const float md = (n & 1) ? da : (da + db) / 2.0f;
+    return (double)md / 0.6745;
+  }
+  const double da = __longlong_as_double((long long)a), db = __longlong_as_double((long long)b);
+  const double md = (n & 1) ? da : (da + db) / 2.0;
+  return md / 0.6745;
+}
+template <bool FP32>
+__device__ __forceinline__ auto dev_key(double m) {
+  if constexpr (FP32)
+    return KeyDev32{(float)m};
+  else
+    return KeyDev64{m};
+}
+
+// Planes of at most MCAP elements: one block per plane, which reads its plane
+// once into LDS and selects there (LDSRC), and planes of any size where the
+// caller has no workspace: the block reads the plane once per pass.
+// The limit is what a selecting block holds in LDS; above it even two planes
+// are faster split.
+constexpr int MCAP = 32768;  // values kept in LDS by a selecting block (128 KiB of the CU's 160)
+
+template <bool VEC, bool FP32, bool LDSRC>
 __global__ void __launch_bounds__(MT) k_band_mad(const float* __restrict__ planes, long long stride, int n,
                                                  double* __restrict__ mad) {
   __shared__ SelShared sh;
+  __shared__ float buf[LDSRC ? MCAP : 1];
   const float* p = planes + (size_t)blockIdx.x * (size_t)stride;
+  if constexpr (LDSRC) {
+    for (int i = threadIdx.x; i < n; i += MT) buf[i] = p[i];
+    __syncthreads();
+    p = buf;
+  }
   uint64_t a, b;
   block_middle<VEC>(p, n, KeyValue{}, sh, &a, &b);
-  const float fa = f32_unkey((uint32_t)a), fb = f32_unkey((uint32_t)b);
-  double r;
-  if constexpr (FP32) {
-    const float m = (n & 1) ? fa : (fa + fb) / 2.0f;
-    block_middle<VEC>(p, n, KeyDev32{m}, sh, &a, &b);
-    const float da = __uint_as_float((uint32_t)a), db = __uint_as_float((uint32_t)b);
-    const float md = (n & 1) ? da : (da + db) / 2.0f;
-    r = (double)md / 0.6745;
-  } else {
-    const double m = (n & 1) ? (double)fa : ((double)fa + (double)fb) / 2.0;
-    block_middle<VEC>(p, n, KeyDev64{m}, sh, &a, &b);
-    const double da = __longlong_as_double((long long)a), db = __longlong_as_double((long long)b);
-    const double md = (n & 1) ? da : (da + db) / 2.0;
-    r = md / 0.6745;
+  const double m = value_median<FP32>(a, b, n);
+  __syncthreads();
+  block_middle<VEC>(p, n, dev_key<FP32>(m), sh, &a, &b);
+  if (threadIdx.x == 0) mad[blockIdx.x] = dev_mad<FP32>(a, b, n);
+}
+
+// ---- large planes: the passes over the plane split over many blocks -------------
+// One block per plane leaves most CUs idle (49 planes on 256 CUs) and reads the
+// plane ten times through one CU: 447 us for 49 planes of 512^2, 0.12 TB/s.
+// Here each of the two medians takes
+//   k_mad_hist    histogram of the keys' top 12 bits, per block
+//   k_mad_find    one block per plane: the bin of the middle rank
+//   k_mad_hist    the next 11 bits inside that bin; returns at once for a plane
+//                 whose bin already fits the candidate buffer (every band of a
+//                 transform does: a bin is an eighth of an octave)
+//   k_mad_gather  values of the bin to the candidate buffer, and the smallest
+//                 key above the bin
+//   k_mad_select  one block per plane: exact selection among the candidates,
+//                 in LDS
+// so the plane is read twice per median, by all CUs: 92 us for the same
+// planes, bound by the latency of ten short dependent launches (the four
+// streaming ones read 51 MB in 11-15 us each).  The 64-bit deviations
+// are binned by their float rounding, which keeps their order, and compared
+// exactly in the last step.  A plane with more candidates than the buffer
+// takes (more than MCAP elements equal in their leading 23 bits) is selected
+// from global memory by its one block.
+constexpr int HBITS = 12, HBINS = 1 << HBITS;        // first histogram
+constexpr int H2BITS = 11, H2BINS = 1 << H2BITS;     // second
+constexpr int ST = 512;                              // threads of the streaming kernels
+constexpr int SCHUNK = 16384, GCHUNK = 8192;         // elements per block
+static_assert(HBINS == 4 * MT && H2BINS == 2 * MT && ST == MT / 2, "bin scans of the streaming kernels");
+
+struct MadState {
+  uint32_t prefix, rank;    // first bin of the middle rank, and the rank inside it
+  uint32_t rank2;           // the rank inside the final bin
+  uint32_t second, ncand;   // the second histogram was needed; candidates
+  uint32_t pad;
+  double m;                 // out: the median of the values
+};
+
+struct MadPlanes {
+  const float* p;
+  long long stride;
+  int n;
+  MadState* st;    // two per plane: values, deviations
+  float* cand;     // MCAP per plane
+  uint16_t* part;  // a histogram per block of the histogram pass, gh blocks per plane
+  uint64_t* above; // smallest key above the bin, per block of the gather, gg blocks per plane
+  int gh, gg;
+};
+
+// The 32-bit binning key of a stage, and the exact key its order refines to.
+template <int STAGE, bool FP32>
+struct MadKey {
+  double m;
+  __device__ uint64_t exact(float v) const {
+    if constexpr (STAGE == 0) return KeyValue{}(v);
+    return dev_key<FP32>(m)(v);
   }
-  if (threadIdx.x == 0) mad[blockIdx.x] = r;
+  __device__ uint32_t bin(float v) const {
+    if constexpr (STAGE == 0) return f32_key(v);
+    if constexpr (FP32) return __float_as_uint(fabsf(v - (float)m));
+    return __float_as_uint((float)fabs((double)v - m));
+  }
+};
+
+// The bin of `rank` among the plane's bins (NB consecutive ones per thread),
+// summed over its blocks' histograms: every thread finds (bin, elements before
+// it, elements in it) in res.
+template <int NB>
+__device__ __forceinline__ void find_bin_parts(const uint16_t* part, int nparts, uint32_t rank, uint32_t* wsum,
+                                               uint32_t* res) {
+  const int t = threadIdx.x;
+  uint32_t h[NB] = {}, s = 0;
+  using V = __attribute__((ext_vector_type(NB))) uint16_t;
+#pragma unroll 4
+  for (int b = 0; b < nparts; ++b) {
+    const V v = *reinterpret_cast<const V*>(part + (size_t)b * HBINS + NB * t);
+#pragma unroll
+    for (int i = 0; i < NB; ++i) h[i] += v[i];
+  }
+#pragma unroll
+  for (int i = 0; i < NB; ++i) s += h[i];
+  uint32_t inc = s;
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t y = __shfl_up(inc, o, 64);
+    if ((t & 63) >= o) inc += y;
+  }
+  if ((t & 63) == 63) wsum[t >> 6] = inc;
+  __syncthreads();
+  uint32_t before = inc - s;
+  for (int w = 0; w < (t >> 6); ++w) before += wsum[w];
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    if (rank >= before && rank < before + h[i]) {
+      res[0] = NB * t + i;
+      res[1] = before;
+      res[2] = h[i];
+    }
+    before += h[i];
+  }
+  __syncthreads();
+}
+
+// The blocks' histograms go to the workspace whole (16-bit counts: a block has
+// SCHUNK elements) and one block per plane adds them up (k_mad_find).  Adding
+// them with a global atomic per occupied bin, or in the plane's last block to
+// finish (whose fence writes the L2 back in every block), took 137 and 160 us
+// for 49 planes of 512^2.
+template <int STAGE, bool VEC, bool FP32, bool SECOND>
+__global__ void __launch_bounds__(ST) k_mad_hist(MadPlanes io) {
+  constexpr int NB = SECOND ? H2BINS : HBINS;
+  static_assert(SCHUNK < 65536, "16-bit counts");
+  __shared__ uint32_t hist[NB];
+  const MadState* st = io.st + 2 * blockIdx.y + STAGE;
+  if (SECOND && !st->second) return;
+  const MadKey<STAGE, FP32> kf{STAGE ? io.st[2 * blockIdx.y].m : 0.0};
+  const uint32_t prefix = SECOND ? st->prefix : 0;
+  for (int i = threadIdx.x; i < NB; i += ST) hist[i] = 0;
+  __syncthreads();
+  const int at = blockIdx.x * SCHUNK;
+  each_value<VEC, ST>(io.p + (size_t)blockIdx.y * io.stride + at, min(SCHUNK, io.n - at), [&](float v) {
+    const uint32_t key = kf.bin(v);
+    if constexpr (SECOND) {
+      if (key >> (32 - HBITS) == prefix) atomicAdd(&hist[(key >> (32 - HBITS - H2BITS)) & (H2BINS - 1)], 1u);
+    } else {
+      atomicAdd(&hist[key >> (32 - HBITS)], 1u);
+    }
+  });
+  __syncthreads();
+  uint32_t* mine = reinterpret_cast<uint32_t*>(io.part + ((size_t)blockIdx.y * io.gh + blockIdx.x) * HBINS);
+  for (int i = threadIdx.x; i < NB / 2; i += ST) mine[i] = hist[2 * i] | (hist[2 * i + 1] << 16);
+}
+
+// The bin of the plane's middle rank, and the start values of the gather.
+template <int STAGE>
+__global__ void __launch_bounds__(ST) k_mad_find(MadPlanes io) {
+  __shared__ uint32_t wsum[ST / 64], res[3];
+  const uint32_t rank = (uint32_t)((io.n - 1) / 2);
+  find_bin_parts<HBINS / ST>(io.part + (size_t)blockIdx.x * io.gh * HBINS, io.gh, rank, wsum, res);
+  if (threadIdx.x == 0) {
+    MadState* st = io.st + 2 * blockIdx.x + STAGE;
+    st->prefix = res[0];
+    st->rank = rank - res[1];
+    st->second = res[2] > (uint32_t)MCAP;
+    st->ncand = 0;
+  }
+}
+
+template <int STAGE, bool VEC, bool FP32>
+__global__ void __launch_bounds__(ST) k_mad_gather(MadPlanes io) {
+  __shared__ float buf[GCHUNK];
+  __shared__ uint32_t cnt, base;
+  __shared__ uint64_t mn[ST / 64];
+  __shared__ uint32_t wsum[ST / 64], res[3];
+  MadState* st = io.st + 2 * blockIdx.y + STAGE;
+  const MadKey<STAGE, FP32> kf{STAGE ? io.st[2 * blockIdx.y].m : 0.0};
+  uint32_t prefix = st->prefix, rank = st->rank, shift = 32 - HBITS;
+  if (st->second) {
+    find_bin_parts<H2BINS / ST>(io.part + (size_t)blockIdx.y * io.gh * HBINS, io.gh, rank, wsum, res);
+    prefix = (prefix << H2BITS) | res[0];
+    rank -= res[1];
+    shift -= H2BITS;
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) st->rank2 = rank;
+  if (threadIdx.x == 0) cnt = 0;
+  __syncthreads();
+  const int at = blockIdx.x * GCHUNK;
+  uint64_t above = ~0ull;
+  uint32_t abin = ~0u;  // binning key of `above`: exact keys are made only for values not past it
+  each_value<VEC, ST>(io.p + (size_t)blockIdx.y * io.stride + at, min(GCHUNK, io.n - at), [&](float v) {
+    const uint32_t bin = kf.bin(v), b = bin >> shift;
+    if (b > prefix) {
+      if (bin > abin) return;
+      const uint64_t key = kf.exact(v);
+      abin = bin;
+      above = key < above ? key : above;
+    } else if (b == prefix) {
+      buf[atomicAdd(&cnt, 1u)] = v;
+    }
+  });
+  for (int o = 32; o > 0; o >>= 1) {
+    const uint64_t a = shfl_xor64(above, o);
+    above = a < above ? a : above;
+  }
+  if ((threadIdx.x & 63) == 0) mn[threadIdx.x >> 6] = above;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < ST / 64; ++w) above = mn[w] < above ? mn[w] : above;
+    io.above[(size_t)blockIdx.y * io.gg + blockIdx.x] = above;
+  }
+  if (threadIdx.x == 0 && cnt) base = atomicAdd(&st->ncand, cnt);
+  __syncthreads();
+  float* out = io.cand + (size_t)blockIdx.y * MCAP;
+  for (uint32_t i = threadIdx.x; i < cnt; i += ST)
+    if (base + i < (uint32_t)MCAP) out[base + i] = buf[i];
+}
+
+template <int STAGE, bool VEC, bool FP32>
+__global__ void __launch_bounds__(MT) k_mad_select(MadPlanes io, double* __restrict__ mad) {
+  __shared__ SelShared sh;
+  __shared__ float buf[MCAP];
+  MadState* st = io.st + 2 * blockIdx.x + STAGE;
+  const MadKey<STAGE, FP32> kf{STAGE ? io.st[2 * blockIdx.x].m : 0.0};
+  const auto exact = [&](float v) { return kf.exact(v); };
+  const uint32_t nc = st->ncand;
+  const bool two = !(io.n & 1);
+  uint64_t a, b, mn = ~0ull, mx = 0;
+  if (nc <= (uint32_t)MCAP) {
+    const float* c = io.cand + (size_t)blockIdx.x * MCAP;
+    for (uint32_t i = threadIdx.x; i < nc; i += MT) {
+      const float v = c[i];
+      const uint64_t key = exact(v);
+      buf[i] = v;
+      mn = key < mn ? key : mn;
+      mx = key > mx ? key : mx;
+    }
+    block_minmax(mn, mx, sh);
+    // the smallest key above the bin, used if the rank is the bin's last
+    uint64_t above = ~0ull, none = 0;
+    if (two && st->rank2 + 1 == nc) {
+      for (int i = threadIdx.x; i < io.gg; i += MT) {
+        const uint64_t key = io.above[(size_t)blockIdx.x * io.gg + i];
+        above = key < above ? key : above;
+      }
+      block_minmax(above, none, sh);
+    }
+    block_pair<false>(buf, (int)nc, st->rank2, two, above, exact, mn, mx, sh, &a, &b);
+  } else {
+    block_middle<VEC>(io.p + (size_t)blockIdx.x * io.stride, io.n, exact, sh, &a, &b);
+  }
+  if (threadIdx.x == 0) {
+    if constexpr (STAGE == 0)
+      st->m = value_median<FP32>(a, b, io.n);
+    else
+      mad[blockIdx.x] = dev_mad<FP32>(a, b, io.n);
+  }
+}
+
+template <int STAGE, bool VEC, bool FP32>
+void launch_mad_stage(const MadPlanes& io, int nplanes, double* mad, hipStream_t s) {
+  const dim3 gh(io.gh, nplanes), gg(io.gg, nplanes);
+  hipLaunchKernelGGL((k_mad_hist<STAGE, VEC, FP32, false>), gh, dim3(ST), 0, s, io);
+  hipLaunchKernelGGL((k_mad_find<STAGE>), dim3(nplanes), dim3(ST), 0, s, io);
+  hipLaunchKernelGGL((k_mad_hist<STAGE, VEC, FP32, true>), gh, dim3(ST), 0, s, io);
+  hipLaunchKernelGGL((k_mad_gather<STAGE, VEC, FP32>), gg, dim3(ST), 0, s, io);
+  hipLaunchKernelGGL((k_mad_select<STAGE, VEC, FP32>), dim3(nplanes), dim3(MT), 0, s, io, mad);
+}
+
+// VEC: float4 loads, for planes that all start on 16 bytes.
+template <bool VEC, bool FP32>
+void launch_mad(const float* planes, long long stride, int n, int nplanes, double* mad, void* work, hipStream_t s) {
+  if (n <= MCAP) {
+    hipLaunchKernelGGL((k_band_mad<false, FP32, true>), dim3(nplanes), dim3(MT), 0, s, planes, stride, n, mad);
+    return;
+  }
+  if (!work) {
+    hipLaunchKernelGGL((k_band_mad<VEC, FP32, false>), dim3(nplanes), dim3(MT), 0, s, planes, stride, n, mad);
+    return;
+  }
+  // grid.y holds at most 65535 planes
+  const int gh = (n + SCHUNK - 1) / SCHUNK, gg = (n + GCHUNK - 1) / GCHUNK;
+  MadState* st = static_cast<MadState*>(work);
+  float* cand = reinterpret_cast<float*>(st + 2 * (size_t)nplanes);
+  uint16_t* part = reinterpret_cast<uint16_t*>(cand + (size_t)nplanes * MCAP);
+  uint64_t* above = reinterpret_cast<uint64_t*>(part + (size_t)nplanes * gh * HBINS);
+  for (int p0 = 0; p0 < nplanes; p0 += 32768) {
+    const MadPlanes io{planes + (size_t)p0 * stride, stride, n, st + 2 * (size_t)p0, cand + (size_t)p0 * MCAP,
+                       part + (size_t)p0 * gh * HBINS, above + (size_t)p0 * gg, gh, gg};
+    launch_mad_stage<0, VEC, FP32>(io, min(32768, nplanes - p0), mad + p0, s);
+    launch_mad_stage<1, VEC, FP32>(io, min(32768, nplanes - p0), mad + p0, s);
+  }
 }
 
 }  // namespace
 }  // namespace shx
 
-extern "C" int shx_band_mad(const float* planes, long long plane_elems, long long plane_stride, int nplanes,
-                            int arith, double* mad, void* stream) {
+extern "C" size_t shx_band_mad_workspace(long long plane_elems, int nplanes) {
+  using namespace shx;
+  if (plane_elems <= MCAP || nplanes < 1) return 0;
+  const size_t gh = (size_t)((plane_elems + SCHUNK - 1) / SCHUNK), gg = (size_t)((plane_elems + GCHUNK - 1) / GCHUNK);
+  return (size_t)nplanes * (2 * sizeof(MadState) + sizeof(float) * MCAP + sizeof(uint16_t) * HBINS * gh +
+                            sizeof(uint64_t) * gg);
+}
+
+extern "C" int shx_band_mad_ws(const float* planes, long long plane_elems, long long plane_stride, int nplanes,
+                               int arith, double* mad, void* work, size_t work_bytes, void* stream) {
   using namespace shx;
   if (!planes || !mad) return fail(SHX_ERR_ARG, "null pointer");
   if (plane_elems < 1 || plane_elems > 0x7fffffffLL) return fail(SHX_ERR_ARG, "plane size %lld outside [1, 2^31)", plane_elems);
@@ -204,21 +554,23 @@ extern "C" int shx_band_mad(const float* planes, long long plane_elems, long lon
   if (nplanes < 0) return fail(SHX_ERR_ARG, "negative plane count");
   if (arith != SHX_MAD_FP64 && arith != SHX_MAD_FP32) return fail(SHX_ERR_ARG, "unknown arithmetic %d", arith);
   if (nplanes == 0) return SHX_OK;
+  if (work && (work_bytes < shx_band_mad_workspace(plane_elems, nplanes) || (uintptr_t)work % 16))
+    return fail(SHX_ERR_ARG, "workspace of %zu bytes (16-byte aligned, at least %zu)", work_bytes,
+                shx_band_mad_workspace(plane_elems, nplanes));
   const int n = (int)plane_elems;
   const bool vec = ((uintptr_t)planes % 16 == 0) && (plane_stride % 4 == 0);
   hipStream_t s = (hipStream_t)stream;
-  const dim3 g(nplanes), b(MT);
-  if (vec) {
-    if (arith == SHX_MAD_FP32)
-      hipLaunchKernelGGL((k_band_mad<true, true>), g, b, 0, s, planes, plane_stride, n, mad);
-    else
-      hipLaunchKernelGGL((k_band_mad<true, false>), g, b, 0, s, planes, plane_stride, n, mad);
-  } else {
-    if (arith == SHX_MAD_FP32)
-      hipLaunchKernelGGL((k_band_mad<false, true>), g, b, 0, s, planes, plane_stride, n, mad);
-    else
-      hipLaunchKernelGGL((k_band_mad<false, false>), g, b, 0, s, planes, plane_stride, n, mad);
-  }
+  if (arith == SHX_MAD_FP32)
+    vec ? launch_mad<true, true>(planes, plane_stride, n, nplanes, mad, work, s)
+        : launch_mad<false, true>(planes, plane_stride, n, nplanes, mad, work, s);
+  else
+    vec ? launch_mad<true, false>(planes, plane_stride, n, nplanes, mad, work, s)
+        : launch_mad<false, false>(planes, plane_stride, n, nplanes, mad, work, s);
   SHX_HIP(hipGetLastError());
   return SHX_OK;
+}
+
+extern "C" int shx_band_mad(const float* planes, long long plane_elems, long long plane_stride, int nplanes,
+                            int arith, double* mad, void* stream) {
+  return shx_band_mad_ws(planes, plane_elems, plane_stride, nplanes, arith, mad, nullptr, 0, stream);
 }

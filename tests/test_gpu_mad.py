@@ -130,3 +130,30 @@ def test_scalars_3d_on_device(gpu):
         plan.close()
     assert np.array_equal(est, np.array(want))
     assert low == want_low
+
+
+@pytest.mark.parametrize("n", [32767, 32768, 32769, 49153, 262147])
+@pytest.mark.parametrize("kind", ["offset", "grid", "halves", "spike", "normal"])
+def test_band_mad_split_planes(gpu, n, kind):
+    """Around the size from which a plane is split over several workgroups:
+    values whose middle bin overflows the first histogram (a narrow band of
+    values on an offset), equal values beyond the candidate buffer (an integer
+    grid; two halves, where the middle pair straddles two bins), and a bin of
+    more distinct values than the buffer holds (a dense spike)."""
+    from shearcuda_amd import api
+    rng = np.random.default_rng(n)
+    a = rng.standard_normal((3, n))
+    if kind == "offset":
+        a = 140.0 + a
+    elif kind == "grid":
+        a = np.round(a * 2)
+    elif kind == "halves":
+        a = np.where(np.arange(n) % 2 == 0, -2.0, 1.0) * np.ones((3, 1))
+    elif kind == "spike":  # 4096 consecutive floats share the leading 12 bits of their keys
+        a = np.float32(1.0) + np.float32(2.0 ** -23) * rng.integers(0, 4096, (3, n)).astype(np.float32)
+    a = a.astype(np.float32)
+    t = torch.from_numpy(a).cuda()
+    for arith, ref in (("fp64", _mad64), ("fp32", _mad32)):
+        got = api.band_mad_cuda(t, arith).cpu().numpy()
+        want = np.array([ref(r) for r in a])
+        assert np.array_equal(got, want), (arith, got, want)
