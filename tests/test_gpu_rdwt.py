@@ -77,3 +77,22 @@ def test_rdwt_adjoints_dense(api):
     ylb, yhb = api.mirdwt_adjoint_cuda(g(Q.reshape(8, m, n)), h, L)
     got = np.concatenate([ylb.cpu().numpy().reshape(8, N), yhb.cpu().numpy().reshape(8, -1)], axis=1)
     assert relmax(got, Q @ S) < 1e-5
+
+
+@pytest.mark.parametrize("name,par", [("Haar", 0), ("Daubechies", 4), ("Daubechies", 6), ("Symmlet", 4)])
+@pytest.mark.parametrize("shape,L", [((8, 8), 3), ((32, 64), 5), ((20, 516), 2), ((36, 1044), 2), ((6, 510), 1),
+                                     ((64, 1536), 5), ((144, 96), 4)])
+def test_rdwt_ragged_shapes(api, name, par, shape, L):
+    """Sides around the level kernels' tiles: rows of at most 512 columns in
+    one block and longer ones split, strips that end inside a tile, dilations
+    longer than the image, every filter length."""
+    from shearcuda_amd.wavelets import MakeONFilter
+    h = MakeONFilter(name, par)
+    x = np.random.default_rng(L).standard_normal((2,) + shape) * 50
+    yl, yh = api.mrdwt_cuda(g(x), h, L)
+    xr = api.mirdwt_cuda(yl, yh, h, L).cpu().numpy()
+    for i in range(2):
+        ryl, ryh = w.mrdwt(x[i], h, L)
+        assert relmax(yl[i].cpu().numpy(), ryl) < 1e-5
+        assert relmax(yh[i].cpu().numpy(), ryh) < 1e-5
+        assert relmax(xr[i], x[i]) < 1e-5
