@@ -24,6 +24,7 @@
 
 #include "api_err.h"
 #include "dict_dev.h"
+#include "spectral.h"
 
 namespace shx {
 namespace {
@@ -85,19 +86,19 @@ __global__ void __launch_bounds__(ST) k_spec_cols(const double2* __restrict__ G,
   for (int k = 0; k < D; ++k) {
     const double2 h = col_dft(G + k * gk, n1, NC, v, u, L, s, tw);
     const double hx = h.x / d0, hy = h.y / d0;
-    float2* mk = main_out + (size_t)k * L * N + (size_t)u * N;
+    float2* mk = main_out + (size_t)k * L * N;
     if (v == 0) {
       const double2 g = col_dft(G + k * gk, n1, NC, N, u, L, s, tw);
       const double gx = g.x / dn, gy = g.y / dn;
       const double ax = 0.5 * (hx + gx) * sc, ay = 0.5 * (hy + gy) * sc;
       const double bx = 0.5 * (hx - gx) * sc, by = 0.5 * (hy - gy) * sc;
       ok = ok && isfinite(ax) && isfinite(ay) && isfinite(bx) && isfinite(by);
-      mk[0] = make_float2((float)ax, (float)ay);
+      mk[sp_ix(L, u, 0)] = make_float2((float)ax, (float)ay);
       beta_out[(size_t)k * L + u] = make_float2((float)bx, (float)by);
     } else {
       const double px = hx * sc, py = hy * sc;
       ok = ok && isfinite(px) && isfinite(py);
-      mk[v] = make_float2((float)px, (float)py);
+      mk[sp_ix(L, u, v)] = make_float2((float)px, (float)py);
     }
   }
   if (!ok) bad[0] = 1;

@@ -103,6 +103,8 @@ void scale_spectra_fp64(int L, int D, int n1, const double* w, int shift, std::v
 void pack_spectra_fp32(int L, int D, const std::vector<std::complex<double>>& H, float* main_out, float* beta_out) {
   const int N = L / 2, NC = N + 1;
   const double sc = 1.0 / ((double)L * (double)L);
+  // strips of 4 columns, as the kernels' sp_ix
+  const auto at = [&](int u, int v) { return (((size_t)(v >> 2) * L + u) * 4 + (v & 3)) * 2; };
   for (int k = 0; k < D; ++k) {
     const cd* Hk = H.data() + (size_t)k * L * NC;
     float* mk = main_out + (size_t)k * L * N * 2;
@@ -110,14 +112,14 @@ void pack_spectra_fp32(int L, int D, const std::vector<std::complex<double>>& H,
     for (int u = 0; u < L; ++u) {
       const cd h0 = Hk[(size_t)u * NC], hn = Hk[(size_t)u * NC + N];
       const cd alpha = 0.5 * (h0 + hn) * sc, beta = 0.5 * (h0 - hn) * sc;
-      mk[((size_t)u * N) * 2 + 0] = (float)alpha.real();
-      mk[((size_t)u * N) * 2 + 1] = (float)alpha.imag();
+      mk[at(u, 0) + 0] = (float)alpha.real();
+      mk[at(u, 0) + 1] = (float)alpha.imag();
       bk[(size_t)u * 2 + 0] = (float)beta.real();
       bk[(size_t)u * 2 + 1] = (float)beta.imag();
       for (int v = 1; v < N; ++v) {
         const cd h = Hk[(size_t)u * NC + v] * sc;
-        mk[((size_t)u * N + v) * 2 + 0] = (float)h.real();
-        mk[((size_t)u * N + v) * 2 + 1] = (float)h.imag();
+        mk[at(u, v) + 0] = (float)h.real();
+        mk[at(u, v) + 1] = (float)h.imag();
       }
     }
   }

@@ -5,6 +5,14 @@
 
 namespace shx {
 
+// Element (row u, column v) of a packed spectrum plane of side L (L rows of
+// L/2 complex values): strips of 4 columns, row by row within a strip.
+template <int L>
+__host__ __device__ __forceinline__ size_t sp_ix(int u, int v) {
+  return (size_t)(((v >> 2) * L + u) * 4 + (v & 3));
+}
+inline __host__ __device__ size_t sp_ix(int L, int u, int v) { return (size_t)(((v >> 2) * L + u) * 4 + (v & 3)); }
+
 // A set of planes spread over up to SHX_MAX_SCALES+1 base pointers ("cells"):
 // plane p of image b lives in cell j with off[j] <= p < off[j+1], at
 //   cell[j] + (p - off[j]) * plane_elems + b * img_stride.
