@@ -212,9 +212,24 @@ int directional(shx3_plan* p, const float* subs, const float* th, float* bands, 
     int rc = fwd3(d, p, subs + v.sub_off, d->sub_total, n, N, 0, p->S, p->sS, nv, s);
     if (rc) return rc;
     const long long fstr = spec_elems(N), n3 = (long long)n * n * n;
+    const float scale = (float)(1.0 / ((double)N * N * N));
+    if (mode == 1 && p->plane_cols < 0 && shx::slab3_supported(N, n, o)) {
+      // rows into slabs (tB), the slabs' other two axes with threshold and sum
+      // (accumulators in tA), one transpose per level
+      const int ns = shx::slab3_splits(n, p->G);
+      const long long slab = (long long)H * N, ass = n3 / 2;
+      for (int g0 = 0; g0 < v.nb; g0 += p->G) {
+        const int G = std::min(p->G, v.nb - g0);
+        shx::Rows3Mul rs{p->S, p->sS, v.F + (size_t)g0 * fstr, fstr, scale, p->tB, 0, n * slab, p->sB, n, o, H * N, G};
+        SHX_LAUNCH(shx::launch3_rows_slab(N, rs, nv, tw, s));
+        shx::Slab3 sl{p->tB, n * slab, p->sB, p->tA, ass, p->sA, th, d->nbands, v.band0 + g0, G, ns, g0 == 0, n, o};
+        SHX_LAUNCH(shx::launch3_slab(N, sl, nv, tw, s));
+      }
+      SHX_LAUNCH(shx::launch3_slab_out(p->tA, ass, p->sA, ns, rec + v.sub_off, d->sub_total, n, nv, s));
+      continue;
+    }
     for (int g0 = 0; g0 < v.nb; g0 += p->G) {
       const int G = std::min(p->G, v.nb - g0);
-      const float scale = (float)(1.0 / ((double)N * N * N));
       if (p->plane_cols >= 0 && shx::plane3_supported(N, n)) {
         // rows and cols of each plane in one kernel, straight into tA
         shx::Plane3Inv pi{p->S, p->sS, v.F + (size_t)g0 * fstr, fstr, scale, p->tA, (long long)H * n * n, p->sA,

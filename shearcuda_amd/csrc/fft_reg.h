@@ -11,7 +11,7 @@
 // a transform split as (R2, R1).  A forward transform, a pointwise product and
 // an inverse transform therefore chain in registers.
 //
-// The short DFTs (2, 3, 4, 5, 8, 9, 16, 32) are fully unrolled with compile-time
+// The short DFTs (2, 3, 4, 5, 6, 8, 9, 10, 12, 16, 32) are fully unrolled with compile-time
 // twiddles (computed below by constexpr series in FP64, rounded once to FP32);
 // the pass twiddles w_N^m come from a table computed in FP64 on the host.
 #pragma once
@@ -139,6 +139,12 @@ __device__ __forceinline__ void dft(float2* v) {
     dft_direct<5, DIR>(v);
   } else if constexpr (R == 9) {
     dft_split<3, 3, DIR>(v);
+  } else if constexpr (R == 6) {
+    dft_split<2, 3, DIR>(v);
+  } else if constexpr (R == 10) {
+    dft_split<2, 5, DIR>(v);
+  } else if constexpr (R == 12) {
+    dft_split<3, 4, DIR>(v);
   } else if constexpr (R == 2) {
     dft2<DIR>(v[0], v[1]);
   } else if constexpr (R == 4) {

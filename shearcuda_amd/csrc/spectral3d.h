@@ -44,6 +44,26 @@ struct Rows3Mul {
   int nlines, G;
 };
 
+// launch3_rows_slab writes the same rows slab by slab (slab j2 = output index
+// along axis 2): element (line, j2) of band g at out + g*out_gs + b*out_bs +
+// j2*nlines + line, lines in the order (k0, k1) of S; out_ld is not used.
+
+// Inverse along axes 1 and 0 of the slabs of G bands, hard threshold (keep
+// |v| > th[b*th_bs + th0 + g]) and sum over the bands of one split: split s of
+// nsplit takes bands s, s + nsplit, ...  acc (split stride acc_ss): slab j2,
+// pair e of axis-1 columns, axis-0 index i0 at ((j2*n/2 + e)*n + i0) as (2e,
+// 2e+1); first = 1 writes it, first = 0 adds to it.
+struct Slab3 {
+  const float2* in;
+  long long in_gs, in_bs;
+  float2* acc;
+  long long acc_ss, acc_bs;
+  const float* th;
+  long long th_bs;
+  int th0, G, nsplit, first;
+  int n, o;
+};
+
 // Fused inverse of one half-spectrum plane for G bands: plane k0 of
 // F_g . S * scale is inverse transformed along axis 2 (rows) and axis 1
 // (cols) with the output window [o_out, o_out + n_out) on both, giving
@@ -126,6 +146,15 @@ bool fft3_supported(int N);
 hipError_t launch3_rows(int N, int dir, const Rows3& io, int nb, const float2* tw, hipStream_t s);
 hipError_t launch3_rows_mul(int N, const Rows3Mul& io, int nb, const float2* tw, hipStream_t s);
 hipError_t launch3_rows_cmac(int N, const Rows3Cmac& io, int nb, const float2* tw, hipStream_t s);
+bool slab3_supported(int N, int n, int o);
+// Accumulators a level of side n keeps per volume (independent of the number
+// of volumes, so a batch sums in the order of a single volume).
+int slab3_splits(int n, int G);
+hipError_t launch3_rows_slab(int N, const Rows3Mul& io, int nb, const float2* tw, hipStream_t s);
+hipError_t launch3_slab(int N, const Slab3& io, int nb, const float2* tw, hipStream_t s);
+// out[i0][i1][j2] = the sum of nsplit accumulators (Slab3).
+hipError_t launch3_slab_out(const float2* acc, long long acc_ss, long long acc_bs, int nsplit, float* out,
+                            long long out_bs, int n, int nb, hipStream_t s);
 // cw: output columns per block (64 or 32; 0 = default).
 bool plane3_supported(int N, int n_out);
 hipError_t launch3_plane_inv(int N, const Plane3Inv& io, int nb, int cw, const float2* tw, hipStream_t s);

@@ -379,10 +379,12 @@ __global__ void __launch_bounds__(CT * Split<N>::R2) k3_pencil_inv(Pencil3Inv io
   const int e = blockIdx.x * CT + c;
   const size_t E = io.E;
   const int b = blockIdx.z;
+  // storing form: one band per block
+  const int g0 = io.mode == 0 ? blockIdx.y : 0, g1 = io.mode == 0 ? g0 + 1 : io.G;
   float2 acc[R1];
 #pragma unroll
   for (int k1 = 0; k1 < R1; ++k1) acc[k1] = make_float2(0.f, 0.f);
-  for (int g = 0; g < io.G; ++g) {
+  for (int g = g0; g < g1; ++g) {
     const float t = io.mode == 1 ? io.th[(size_t)b * io.th_bs + io.th0 + g] : 0.0f;
     if (n1 < R1) {
       const float2* src = io.in + (size_t)b * io.in_bs + (size_t)g * io.in_gs + 2 * (size_t)e;
@@ -456,6 +458,394 @@ __global__ void __launch_bounds__(CT * Split<N>::R2) k3_pencil_inv(Pencil3Inv io
       if (in_window(j, io.n_out)) *reinterpret_cast<float2*>(dst + (size_t)j * E) = acc[k1];
     }
   }
+}
+
+// ---------------------------------------------------------------------------
+// Slab form of the thresholded band loop.  After the inverse rows, the other
+// two axes of one output index j2 ("slab") are a half spectrum of (N/2 + 1) x N
+// values: 84 KB at N = 144, which fits a CU's LDS.  k3_rows_band writes the
+// rows slab by slab, and one block of k3_slab inverse transforms a slab along
+// axis 1 and axis 0, thresholds it and keeps the running sum of its bands in
+// registers.  Against separate column and pencil passes, one write and one read
+// of the band spectra (19 of 41 MB per band and volume at 128^3) stay on the
+// chip.  Transforms are N = P * Q two-pass splits with P and Q close, so that
+// (nearly) every lane works in both passes and a line's exchange stays inside
+// one wave.
+// 8 bands of two 128^3 volumes: rows 82 -> 62 us (290 MB: the copy rate), columns
+// and pencils 67 + 50 -> 73 us (172 MB; the block's LDS and vector pipes are each
+// busy half of the time, one after the other: one block per CU).
+template <int N>
+struct Split3;
+template <> struct Split3<24> { static constexpr int P = 4, Q = 6, NP = 12; };
+template <> struct Split3<32> { static constexpr int P = 4, Q = 8, NP = 16; };
+template <> struct Split3<48> { static constexpr int P = 6, Q = 8, NP = 24; };
+template <> struct Split3<64> { static constexpr int P = 8, Q = 8, NP = 32; };
+template <> struct Split3<80> { static constexpr int P = 8, Q = 10, NP = 40; };
+// NP: most axis-1 pairs of a slab.  Sides of at most 128 (64 pairs) leave both
+// LDS tiles inside the CU.
+template <> struct Split3<144> { static constexpr int P = 12, Q = 12, NP = 64; };
+
+template <int N>
+struct Slab3Cfg {
+  static constexpr int P = Split3<N>::P, Q = Split3<N>::Q, NP = Split3<N>::NP;
+  static constexpr int H = N / 2 + 1;
+  static constexpr int LPW = 64 / Q;                       // lines per wave
+  static constexpr int WL = (H + LPW - 1) / LPW, WP = (NP + LPW - 1) / LPW;
+  static constexpr int T = 64 * (WL > WP ? WL : WP);
+  // line stride in LDS: 2 LS mod 64 words is an odd multiple of 4, so the
+  // 16-byte reads down the lines (phase 2) fall on distinct banks
+  static constexpr int LS = N + 2;
+  static_assert(T <= 1024 && P <= Q && Q % 2 == 0, "one round per phase");
+};
+
+// LDS accesses of one wave stay in order; this keeps the compiler from moving
+// them across the exchange.
+__device__ __forceinline__ void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Place of (n1, k2) in a line's exchange.  The second pass reads it at a stride
+// of P over the lanes; where that falls on few banks (multiples of 8 words at
+// P = 12, of 16 at P = 8) a slot is skipped after every four k2.
+template <int P, int Q>
+__device__ __forceinline__ int xch(int n1, int k2) {
+  if constexpr (P == 12 || P == 8)
+    return n1 + P * k2 + k2 / 4;
+  else
+    return n1 + P * k2;
+}
+// First pass of a transform on x[n1 + P n2] (n2 < Q): DFT of length Q,
+// twiddles w_N^(n1 k2) (tws[m] = exp(-2 pi i m / N)), to the exchange.
+template <int P, int Q, int DIR>
+__device__ __forceinline__ void two_first(float2 (&v)[Q], int n1, float2* line, const float2* tws) {
+  dft<Q, DIR>(v);
+  line[xch<P, Q>(n1, 0)] = v[0];
+#pragma unroll
+  for (int k = 1; k < Q; ++k)
+    line[xch<P, Q>(n1, k)] = DIR > 0 ? cmulc(v[k], tws[n1 * k]) : cmul(v[k], tws[n1 * k]);
+}
+// Second pass: X[k2 + Q k1], k1 < P.
+template <int P, int Q, int DIR>
+__device__ __forceinline__ void two_second(float2 (&u)[P], int k2, const float2* line) {
+#pragma unroll
+  for (int a = 0; a < P; ++a) u[a] = line[xch<P, Q>(a, k2)];
+  dft<P, DIR>(u);
+}
+
+// Inverse rows of F_g . S, 16 lines per block, bands [z, z + 1) * gper of the
+// group.  The next band's F is loaded while this band is transformed.  SLAB:
+// outputs leave line-fastest, 128 contiguous bytes per slab; else row by row.
+constexpr int SLAB_LINES = 16;
+template <int N, bool SLAB>
+__global__ void __launch_bounds__(SLAB_LINES * Split3<N>::Q) k3_rows_band(Rows3Mul io, int gper,
+                                                                          const float2* __restrict__ tw) {
+  constexpr int P = Split3<N>::P, Q = Split3<N>::Q, LS = N + 5, T = SLAB_LINES * Q;
+  __shared__ float2 buf[SLAB_LINES * LS];
+  __shared__ float2 tws[N];
+  const int tid = threadIdx.x;
+  for (int i = tid; i < N; i += T) tws[i] = tw[i];
+  // volumes fastest: those of one line block read the same F lines, and run on
+  // one XCD (the low 3 bits of the dispatch order)
+  const int nv = gridDim.y, total = gridDim.x * nv;
+  int id = blockIdx.x + gridDim.x * blockIdx.y;
+  if (total % 8 == 0) id = (id % 8) * (total / 8) + id / 8;
+  const int b = id % nv, line0 = (id / nv) * SLAB_LINES;
+  const int g0 = blockIdx.z * gper, g1 = min(io.G, g0 + gper);
+  const int la = tid / P, n1 = tid % P;
+  const bool vA = la < SLAB_LINES && line0 + la < io.nlines;
+  const int lb = SLAB ? tid % SLAB_LINES : tid / Q, k2 = SLAB ? tid / SLAB_LINES : tid % Q;
+  const bool vB = line0 + lb < io.nlines;
+  float2 sv[Q], f[Q];
+  const float2* F = io.F + (size_t)g0 * io.f_gs + (size_t)(line0 + la) * N + n1;
+  if (vA) {
+    const float2* S = io.S + (size_t)b * io.s_bs + (size_t)(line0 + la) * N + n1;
+#pragma unroll
+    for (int n2 = 0; n2 < Q; ++n2) {
+      sv[n2] = S[P * n2];
+      f[n2] = F[P * n2];
+    }
+#pragma unroll
+    for (int n2 = 0; n2 < Q; ++n2) sv[n2] = cscale(sv[n2], io.scale);
+  }
+  float2* out = io.out + (size_t)b * io.out_bs + (SLAB ? (size_t)(line0 + lb) : (size_t)(line0 + lb) * io.out_ld);
+  const size_t step = SLAB ? io.nlines : 1;
+  __syncthreads();  // tws
+  for (int g = g0; g < g1; ++g) {
+    if (vA) {
+      float2 v[Q];
+#pragma unroll
+      for (int n2 = 0; n2 < Q; ++n2) v[n2] = cmul(sv[n2], f[n2]);
+      if (g + 1 < g1) {
+        F += io.f_gs;
+#pragma unroll
+        for (int n2 = 0; n2 < Q; ++n2) f[n2] = F[P * n2];
+      }
+      two_first<P, Q, +1>(v, n1, buf + la * LS, tws);
+    }
+    __syncthreads();
+    if (vB) {
+      float2 u[P];
+      two_second<P, Q, +1>(u, k2, buf + lb * LS);
+      float2* dst = out + (size_t)g * io.out_gs;
+#pragma unroll
+      for (int k1 = 0; k1 < P; ++k1) {
+        const int j = k2 + Q * k1 - io.o_out;
+        if (in_window(j, io.n_out)) dst[(size_t)j * step] = u[k1];
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// Forward rows of G band inputs times conj(F_g), summed over the group, CMAC_LINES
+// lines per block (k3_rows_cmac on the lane-filling split, with the next band's
+// input and filter lines in flight across the transform).
+constexpr int CMAC_LINES = 8;
+template <int N>
+__global__ void __launch_bounds__(CMAC_LINES * Split3<N>::Q) k3_rows_cmac2(Rows3Cmac io, const float2* __restrict__ tw) {
+  constexpr int P = Split3<N>::P, Q = Split3<N>::Q, LS = N + 5, T = CMAC_LINES * Q;
+  __shared__ float2 buf[CMAC_LINES * LS];
+  __shared__ float2 tws[N];
+  const int tid = threadIdx.x;
+  for (int i = tid; i < N; i += T) tws[i] = tw[i];
+  const int line0 = blockIdx.x * CMAC_LINES;
+  const int la = tid / P, n1 = tid % P;
+  const bool vA = la < CMAC_LINES && line0 + la < io.nlines;
+  const int lb = tid / Q, k2 = tid % Q;
+  const bool vB = line0 + lb < io.nlines;
+  const float2* src = io.in + (size_t)blockIdx.y * io.in_bs + (size_t)(line0 + la) * io.in_ld;
+  const float2* F = io.F + (size_t)(line0 + lb) * N + k2;
+  float2 v[Q], f[P], acc[P];
+#pragma unroll
+  for (int k = 0; k < P; ++k) acc[k] = make_float2(0.f, 0.f);
+  const auto load = [&]() {
+    if (vA) {
+#pragma unroll
+      for (int n2 = 0; n2 < Q; ++n2) {
+        const int j = n1 + P * n2 - io.o_in;
+        v[n2] = in_window(j, io.n_in) ? src[j] : make_float2(0.f, 0.f);
+      }
+    }
+  };
+  load();
+  __syncthreads();  // tws
+  for (int g = 0; g < io.G; ++g) {
+    if (vB) {
+#pragma unroll
+      for (int k = 0; k < P; ++k) f[k] = F[Q * k];
+    }
+    if (vA) two_first<P, Q, -1>(v, n1, buf + la * LS, tws);
+    src += io.in_gs;
+    F += io.f_gs;
+    if (g + 1 < io.G) load();
+    __syncthreads();
+    if (vB) {
+      float2 u[P];
+      two_second<P, Q, -1>(u, k2, buf + lb * LS);
+#pragma unroll
+      for (int k = 0; k < P; ++k) acc[k] = cadd(acc[k], cmulc(u[k], f[k]));
+    }
+    __syncthreads();
+  }
+  if (vB) {
+    float2* dst = io.out + (size_t)blockIdx.y * io.out_bs + (size_t)(line0 + lb) * N + k2;
+#pragma unroll
+    for (int k = 0; k < P; ++k) acc[k] = cscale(acc[k], io.scale);
+    if (io.accumulate) {  // every old value loaded before the first store
+      float2 old[P];
+#pragma unroll
+      for (int k = 0; k < P; ++k) old[k] = dst[Q * k];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < P; ++k) acc[k] = cadd(old[k], acc[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < P; ++k) dst[Q * k] = acc[k];
+  }
+}
+
+// One block per (slab, split, volume); bands in turn.  Phase 1: line k0 along
+// axis 1 (its exchange in its own LDS line).  Phase 2: pair e of axis-1 columns
+// (2e, 2e+1) as one complex pencil along axis 0.  A block of 15 waves fills the
+// CU at N = 144 (one block, 160 KB of LDS); the next band's lines are loaded
+// before phase 2, so their latency hides behind it.
+template <int N>
+__global__ void __launch_bounds__(Slab3Cfg<N>::T) k3_slab(Slab3 io, const float2* __restrict__ tw) {
+  using C = Slab3Cfg<N>;
+  constexpr int P = C::P, Q = C::Q, H = C::H, LS = C::LS;
+  __shared__ __align__(16) float2 U[H * LS];
+  __shared__ float2 Z[C::NP * LS];
+  __shared__ float2 tws[N];
+  const int tid = threadIdx.x, lane = tid & 63, sub = lane / Q, i = lane % Q;
+  const int line = (tid >> 6) * C::LPW + sub;  // k0 in phase 1, the pair in phase 2
+  const int j2 = blockIdx.x, split = blockIdx.y, b = blockIdx.z, n = io.n, np = n / 2;
+  const bool vl = sub < C::LPW && line < H, vp = sub < C::LPW && line < np;
+  for (int k = tid; k < N; k += C::T) tws[k] = tw[k];
+  const float2* src = io.in + (size_t)b * io.in_bs + (size_t)j2 * (H * N) + (size_t)line * N + i;
+  float2 v[Q], acc[P];
+#pragma unroll
+  for (int k = 0; k < P; ++k) acc[k] = make_float2(0.f, 0.f);
+  const auto load = [&](int g) {
+    if (vl && i < P && g < io.G) {
+      const float2* p = src + (size_t)g * io.in_gs;
+#pragma unroll
+      for (int n2 = 0; n2 < Q; ++n2) v[n2] = p[P * n2];
+    }
+  };
+  load(split);
+  __syncthreads();  // tws
+  float2* ul = U + line * LS;
+  float2* zl = Z + line * LS;
+  for (int g = split; g < io.G; g += io.nsplit) {
+    if (vl && i < P) two_first<P, Q, +1>(v, i, ul, tws);
+    wave_order();
+    float2 u[P];
+    if (vl) two_second<P, Q, +1>(u, i, ul);
+    wave_order();
+    if (vl) {
+#pragma unroll
+      for (int k1 = 0; k1 < P; ++k1) ul[i + Q * k1] = u[k1];  // the whole line: phase 2 reads its window
+    }
+    load(g + io.nsplit);
+    const float t = io.th[(size_t)b * io.th_bs + io.th0 + g];
+    __syncthreads();  // the slab's columns are complete
+    float2 z[Q];
+    if (vp && i < P) {
+#pragma unroll
+      for (int n2 = 0; n2 < Q; ++n2) {
+        // m = i + P n2 < N/2 exactly for n2 < Q/2
+        const int km = n2 < Q / 2 ? i + P * n2 : N - P * n2 - i;
+        const float4 ab = *reinterpret_cast<const float4*>(U + km * LS + io.o + 2 * line);
+        // Z[m] = A[m] + i B[m]; Z[N-m] = conj(A[m]) + i conj(B[m]); the
+        // imaginary parts at m = 0 and N/2 are dropped as in a real inverse.
+        z[n2] = n2 < Q / 2 ? make_float2(ab.x - ab.w, ab.y + ab.z) : make_float2(ab.x + ab.w, ab.z - ab.y);
+        if (n2 == 0 || n2 == Q / 2)
+          if (i == 0) z[n2] = make_float2(ab.x, ab.z);
+      }
+    }
+    __syncthreads();  // the next band may overwrite the columns
+    if (vp && i < P) two_first<P, Q, +1>(z, i, zl, tws);
+    wave_order();
+    if (vp) {
+      two_second<P, Q, +1>(u, i, zl);
+#pragma unroll
+      for (int k1 = 0; k1 < P; ++k1)
+        acc[k1] = cadd(acc[k1], make_float2(hard_keep(u[k1].x, t), hard_keep(u[k1].y, t)));
+    }
+    wave_order();
+  }
+  if (vp) {
+    float2* a = io.acc + (size_t)b * io.acc_bs + (size_t)split * io.acc_ss + ((size_t)j2 * np + line) * n;
+    if (!io.first) {  // every old value loaded before the first store
+      float2 old[P];
+#pragma unroll
+      for (int k1 = 0; k1 < P; ++k1) {
+        const int j = i + Q * k1 - io.o;
+        old[k1] = in_window(j, n) ? a[j] : make_float2(0.f, 0.f);
+      }
+#pragma unroll
+      for (int k1 = 0; k1 < P; ++k1) acc[k1] = cadd(old[k1], acc[k1]);
+    }
+#pragma unroll
+    for (int k1 = 0; k1 < P; ++k1) {
+      const int j = i + Q * k1 - io.o;
+      if (in_window(j, n)) a[j] = acc[k1];
+    }
+  }
+}
+
+// Sum of the splits' accumulators, transposed to (i0, i1, j2): a block takes
+// one pair of axis-1 columns and a tile of 32 x 32 (j2, i0).
+__global__ void __launch_bounds__(256) k3_slab_out(const float2* __restrict__ acc, long long ss, long long bs, int nsplit,
+                                                   float* __restrict__ out, long long obs, int n) {
+  __shared__ float2 t[32][33];
+  const int np = n / 2, e = blockIdx.y, b = blockIdx.z, nt = (n + 31) / 32;
+  const int j0 = (blockIdx.x / nt) * 32, i0 = (blockIdx.x % nt) * 32;
+  const int x = threadIdx.x & 31, y = threadIdx.x >> 5;
+  const float2* a = acc + (size_t)b * bs;
+#pragma unroll
+  for (int r = 0; r < 32; r += 8) {
+    const int j = j0 + y + r, i = i0 + x;
+    float2 s = make_float2(0.f, 0.f);
+    if (j < n && i < n)
+      for (int k = 0; k < nsplit; ++k) s = cadd(s, a[(size_t)k * ss + ((size_t)j * np + e) * n + i]);
+    t[y + r][x] = s;
+  }
+  __syncthreads();
+  float* o = out + (size_t)b * obs;
+#pragma unroll
+  for (int r = 0; r < 32; r += 8) {
+    const int i = i0 + y + r, j = j0 + x;
+    if (i < n && j < n) {
+      const float2 s = t[x][y + r];
+      o[((size_t)i * n + 2 * e) * n + j] = s.x;
+      o[((size_t)i * n + 2 * e + 1) * n + j] = s.y;
+    }
+  }
+}
+
+// A block runs all bands of its lines (the spectrum S is then read once) unless
+// that leaves fewer than 1024 blocks (4 per CU): the small levels' launches were
+// chains of 8 transforms in 205 blocks (80^3 grid: 16.6 us per group of 8, split
+// 11.3 us).
+template <int N, bool SLAB>
+static hipError_t rows_band_n(const Rows3Mul& io, int nb, const float2* tw, hipStream_t s) {
+  const int nl = (io.nlines + SLAB_LINES - 1) / SLAB_LINES;
+  int gper = io.G;
+  while (gper > 1 && nl * nb * ((io.G + gper - 1) / gper) < 1024) gper = (gper + 1) / 2;
+  hipLaunchKernelGGL((k3_rows_band<N, SLAB>), dim3(nl, nb, (io.G + gper - 1) / gper), dim3(SLAB_LINES * Split3<N>::Q), 0,
+                     s, io, gper, tw);
+  return hipGetLastError();
+}
+template <int N>
+static hipError_t rows_cmac2_n(const Rows3Cmac& io, int nb, const float2* tw, hipStream_t s) {
+  hipLaunchKernelGGL((k3_rows_cmac2<N>), dim3((io.nlines + CMAC_LINES - 1) / CMAC_LINES, nb),
+                     dim3(CMAC_LINES * Split3<N>::Q), 0, s, io, tw);
+  return hipGetLastError();
+}
+template <int N>
+static hipError_t slab_n(const Slab3& io, int nb, const float2* tw, hipStream_t s) {
+  hipLaunchKernelGGL((k3_slab<N>), dim3(io.n, io.nsplit, nb), dim3(Slab3Cfg<N>::T), 0, s, io, tw);
+  return hipGetLastError();
+}
+#define SHX3_SLAB_BY_N(N, F)          \
+  switch (N) {                        \
+    case 24: return F(24);            \
+    case 32: return F(32);            \
+    case 48: return F(48);            \
+    case 64: return F(64);            \
+    case 80: return F(80);            \
+    case 144: return F(144);          \
+    default: return hipErrorInvalidValue; \
+  }
+bool slab3_supported(int N, int n, int o) {
+  switch (N) {
+    case 24: case 32: case 48: case 64: case 80: return n % 2 == 0 && n + o <= N && o % 2 == 0;
+    case 144: return n % 2 == 0 && n <= 128 && n + o <= N && o % 2 == 0;
+    default: return false;
+  }
+}
+int slab3_splits(int n, int G) {
+  int s = 1;  // 128: two splits, a block for every CU; small sides, whose blocks share a CU, up to 8
+  while (s < 8 && 2 * s <= G && n * s < 256) s *= 2;
+  return s;
+}
+hipError_t launch3_rows_slab(int N, const Rows3Mul& io, int nb, const float2* tw, hipStream_t s) {
+#define F(M) rows_band_n<M, true>(io, nb, tw, s)
+  SHX3_SLAB_BY_N(N, F)
+#undef F
+}
+hipError_t launch3_slab(int N, const Slab3& io, int nb, const float2* tw, hipStream_t s) {
+#define F(M) slab_n<M>(io, nb, tw, s)
+  SHX3_SLAB_BY_N(N, F)
+#undef F
+}
+hipError_t launch3_slab_out(const float2* acc, long long acc_ss, long long acc_bs, int nsplit, float* out,
+                            long long out_bs, int n, int nb, hipStream_t s) {
+  const int nt = (n + 31) / 32;
+  hipLaunchKernelGGL(k3_slab_out, dim3(nt * nt, n / 2, nb), dim3(256), 0, s, acc, acc_ss, acc_bs, nsplit, out, out_bs, n);
+  return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
@@ -585,7 +975,7 @@ struct Launch3 {
   }
   template <int CT>
   static hipError_t pinv_ct(const Pencil3Inv& io, int nb, const float2* tw, hipStream_t s) {
-    const dim3 grid(io.E / 2 / CT, 1, nb);
+    const dim3 grid(io.E / 2 / CT, io.mode == 0 ? io.G : 1, nb);
     hipLaunchKernelGGL((k3_pencil_inv<N, CT>), grid, dim3(Cols3Cfg<N, CT>::T), 0, s, io, tw);
     return hipGetLastError();
   }
@@ -621,10 +1011,32 @@ hipError_t launch3_rows(int N, int dir, const Rows3& io, int nb, const float2* t
   SHX3_BY_N(N, LT::rows(dir, io, nb, tw, s))
 }
 hipError_t launch3_rows_mul(int N, const Rows3Mul& io, int nb, const float2* tw, hipStream_t s) {
-  SHX3_BY_N(N, LT::rows_mul(io, nb, tw, s))
+  switch (N) {
+    case 24: return rows_band_n<24, false>(io, nb, tw, s);
+    case 32: return rows_band_n<32, false>(io, nb, tw, s);
+    case 48: return rows_band_n<48, false>(io, nb, tw, s);
+    case 64: return rows_band_n<64, false>(io, nb, tw, s);
+    case 80: return rows_band_n<80, false>(io, nb, tw, s);
+    case 144: return rows_band_n<144, false>(io, nb, tw, s);
+    case 8: return Launch3<8>::rows_mul(io, nb, tw, s);
+    case 16: return Launch3<16>::rows_mul(io, nb, tw, s);
+    case 128: return Launch3<128>::rows_mul(io, nb, tw, s);
+    default: return hipErrorInvalidValue;
+  }
 }
 hipError_t launch3_rows_cmac(int N, const Rows3Cmac& io, int nb, const float2* tw, hipStream_t s) {
-  SHX3_BY_N(N, LT::rows_cmac(io, nb, tw, s))
+  switch (N) {
+    case 24: return rows_cmac2_n<24>(io, nb, tw, s);
+    case 32: return rows_cmac2_n<32>(io, nb, tw, s);
+    case 48: return rows_cmac2_n<48>(io, nb, tw, s);
+    case 64: return rows_cmac2_n<64>(io, nb, tw, s);
+    case 80: return rows_cmac2_n<80>(io, nb, tw, s);
+    case 144: return rows_cmac2_n<144>(io, nb, tw, s);
+    case 8: return Launch3<8>::rows_cmac(io, nb, tw, s);
+    case 16: return Launch3<16>::rows_cmac(io, nb, tw, s);
+    case 128: return Launch3<128>::rows_cmac(io, nb, tw, s);
+    default: return hipErrorInvalidValue;
+  }
 }
 bool plane3_supported(int N, int n_out) { return N >= 24 && fft3_supported(N) && n_out >= 8; }
 

@@ -261,3 +261,38 @@ def test_identity_and_lowpass_at_128(mods):
     want = plan.pyr_rec(subs)
     assert float((out2 - want).abs().max() / want.abs().max()) < TOL
     plan.close()
+
+
+@pytest.mark.parametrize("n,group,dirs,mode", [(32, 1, (4, 3, 2), 1), (48, 3, (4, 3, 2), 1.5), (64, 5, (4, 2, 2), 1),
+                                               (64, 8, (3, 2, 2), 2), (128, 7, (3, 2, 2), 1)])
+def test_slab_band_loop_equals_bands(mods, n, group, dirs, mode):
+    """The band loop that keeps a slab in LDS (every FFT grid it covers, groups
+    that do not divide the band count, more splits than bands left in a group)
+    against the materialised bands, thresholded and summed; thresholds lie in
+    a gap of each band's magnitudes."""
+    print("case slab n=%d" % n, flush=True)
+    sh = mods[1].Shear3D(n, dirs, mode)
+    plan = mods[1].Plan3D(sh, 2, group=group)
+    x = torch.tensor(_vol(n, 71, nvol=2), dtype=torch.float32, device="cuda")
+    subs = plan.pyr_dec(x)
+    lev = sh.split_bands(plan.analysis(subs))
+    th = torch.empty(2, sh.nbands, device="cuda")
+    want = []
+    for l, b in enumerate(lev):
+        m = b.abs().reshape(2, b.shape[1], -1)
+        k0 = sh.band_first[l]
+        for v in range(2):
+            for k in range(b.shape[1]):
+                s = torch.sort(m[v, k]).values
+                h = s.numel()
+                w = s[h // 2:h // 2 + h // 4]
+                i = int(torch.argmax(w[1:] - w[:-1]))
+                th[v, k0 + k] = 0.5 * (w[i] + w[i + 1])
+        t = th[:, k0:k0 + b.shape[1], None, None, None]
+        want.append(torch.where(b.abs() > t, b, torch.zeros_like(b)).double().sum(1))
+    rec = plan.dec_thresh_rec(subs, th)
+    for l, (got, ref) in enumerate(zip(sh.split_subs(rec), want)):
+        err = float((got.double() - ref).abs().max() / ref.abs().max())
+        assert err < TOL, (l, err)
+    plan.close()
+    sh.close()
