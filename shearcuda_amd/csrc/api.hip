@@ -428,7 +428,9 @@ void set_group(const shx_dict* d, Work& w, int g) {
 
 int alloc_work(const shx_dict* d, int nimg, Work& w) {
   const long long pl = (long long)d->L * d->L;
-  set_group(d, w, nimg == 1 ? 4 : 4);
+  // the same groups for every number of images: a batch then sums each scale's
+  // directions in the order of a single image, with the same bits
+  set_group(d, w, 4);
   w.s_planes = pl * (d->S + 3);
   w.s_spec = pl * d->S;
   w.s_band = pl * d->nbands;

@@ -1163,9 +1163,9 @@ __global__ void __launch_bounds__(CT * 64) k_cols_dec3(const float2* __restrict_
                                                    float2* __restrict__ Tout, long long t_stride,
                                                    const float2* __restrict__ Hmain, const float2* __restrict__ Hbeta,
                                                    BandMap map, const float2* __restrict__ tw) {
-  static_assert(L == 512, "three-pass engine: 512 points");
-  using E = Col3<CT>;
-  constexpr int NH = L / 2;
+  using G = ColEng<L, CT>;
+  using E = typename G::E;
+  constexpr int NH = L / 2, NV = G::NV;
   __shared__ float2 buf[E::LDS];
   int tile, slot, b;
   col_block_order_lines<(16 / CT > 1 ? 16 / CT : 1)>(tile, slot, b);
@@ -1177,31 +1177,31 @@ __global__ void __launch_bounds__(CT * 64) k_cols_dec3(const float2* __restrict_
   const BufView xv = col_view<L, CT>(src);
   const BufView hv = col_view<L, CT>(Hmain + (size_t)f * L * NH + sp_ix<L>(0, c0));
   const unsigned lane = col_off<L>(tau, c);
-  float2 x[8], h[8];
+  float2 x[NV], h[NV];
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
+  for (int k = 0; k < NV; ++k) {
     x[k] = xv.ld2(lane, col_off<L>(64 * k, 0));
     h[k] = hv.ld2(lane, col_off<L>(64 * k, 0));
   }
-  const Fft3Tw t = fft3_tw(tau, tw);
+  const typename G::Tw t = G::twiddles(tau, tw);
   __builtin_amdgcn_sched_barrier(0);  // data, filter and twiddle loads in flight together
-  float2 q[8];
+  float2 q[NV];
 #pragma unroll
-  for (int k = 0; k < 8; ++k) q[k] = cmul(h[k], x[k]);
+  for (int k = 0; k < NV; ++k) q[k] = cmul(h[k], x[k]);
   if (c0 == 0 && c == 0) {
     // packed (DC, Nyquist) column: + beta(u) conj(X(-u))
     const float2* hb = Hbeta + (size_t)f * L;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
+    for (int k = 0; k < NV; ++k) {
       const int u = tau + 64 * k;
       const float2 pm = cconj(src[sp_ix<L>((L - u) & (L - 1), 0)]);
       q[k] = cadd(q[k], cmul(hb[u], pm));
     }
   }
-  fft512_3<CT, +1>(q, buf, t);
+  G::template fft<+1>(q, buf, t);
   const BufView tv = col_view<L, CT>(Tout + (size_t)b * t_stride + (size_t)p * L * NH + sp_ix<L>(0, c0));
 #pragma unroll
-  for (int k = 0; k < 8; ++k) tv.st2(q[k], lane, col_off<L>(64 * k, 0));
+  for (int k = 0; k < NV; ++k) tv.st2(q[k], lane, col_off<L>(64 * k, 0));
 }
 
 template <int L, int CT>
@@ -1209,9 +1209,9 @@ __global__ void __launch_bounds__(CT * 64) k_cols_rec3(const float2* __restrict_
                                                    float2* __restrict__ Q, long long q_stride,
                                                    const float2* __restrict__ Hmain, const float2* __restrict__ Hbeta,
                                                    BandMap map, const float2* __restrict__ tw) {
-  static_assert(L == 512, "three-pass engine: 512 points");
-  using E = Col3<CT>;
-  constexpr int NH = L / 2;
+  using G = ColEng<L, CT>;
+  using E = typename G::E;
+  constexpr int NH = L / 2, NV = G::NV;
   __shared__ float2 buf[E::LDS];
   int tile, slot, b;
   if (gridDim.z == 1)  // one image: 29.3 -> 26.9 us at 4 columns
@@ -1224,47 +1224,59 @@ __global__ void __launch_bounds__(CT * 64) k_cols_rec3(const float2* __restrict_
   const int p0 = map_u16(map.group_band0, g), p1 = map_u16(map.group_band0, g + 1);
   const float2* ub = U + (size_t)b * u_stride + sp_ix<L>(0, c0);
   const unsigned lane = col_off<L>(tau, c);
-  const Fft3Tw t = fft3_tw(tau, tw);
-  float2 acc[8];
+  const typename G::Tw t = G::twiddles(tau, tw);
+  float2 acc[NV];
 #pragma unroll
-  for (int k = 0; k < 8; ++k) acc[k] = make_float2(0.f, 0.f);
+  for (int k = 0; k < NV; ++k) acc[k] = make_float2(0.f, 0.f);
   // software pipeline: the band tile of the next direction is loaded while
   // this direction is transformed (the filter tile is already in flight
   // across the transform: it is used last)
-  float2 vn[8];
-  {
+  constexpr bool ahead = NV <= 8;
+  float2 vn[NV];
+  if constexpr (ahead) {
     const BufView uv = col_view<L, CT>(ub + (size_t)p0 * L * NH);
 #pragma unroll
-    for (int k = 0; k < 8; ++k) vn[k] = uv.ld2(lane, col_off<L>(64 * k, 0));
+    for (int k = 0; k < NV; ++k) vn[k] = uv.ld2(lane, col_off<L>(64 * k, 0));
   }
   for (int p = p0; p < p1; ++p) {
     const int f = map_u8(map.filt_of, p);
     const BufView hv = col_view<L, CT>(Hmain + (size_t)f * L * NH + sp_ix<L>(0, c0));
-    float2 v[8], h[8];
+    float2 v[NV], h[NV];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      v[k] = vn[k];
-      h[k] = hv.ld2(lane, col_off<L>(64 * k, 0));
+    for (int k = 0; k < NV; ++k) {
+      if constexpr (ahead) {
+        v[k] = vn[k];
+        h[k] = hv.ld2(lane, col_off<L>(64 * k, 0));
+      }
     }
-    if (p + 1 < p1) {
+    if constexpr (!ahead) {
+      const BufView uv = col_view<L, CT>(ub + (size_t)p * L * NH);
+#pragma unroll
+      for (int k = 0; k < NV; ++k) v[k] = uv.ld2(lane, col_off<L>(64 * k, 0));
+    }
+    if (ahead && p + 1 < p1) {
       const BufView uv = col_view<L, CT>(ub + (size_t)(p + 1) * L * NH);
 #pragma unroll
-      for (int k = 0; k < 8; ++k) vn[k] = uv.ld2(lane, col_off<L>(64 * k, 0));
+      for (int k = 0; k < NV; ++k) vn[k] = uv.ld2(lane, col_off<L>(64 * k, 0));
     }
     __builtin_amdgcn_sched_barrier(0);
     if (p > p0) __syncthreads();  // the previous direction's reads of buf are complete
-    fft512_3<CT, -1>(v, buf, t);
+    G::template fft<-1>(v, buf, t);
+    if constexpr (!ahead) {
+#pragma unroll
+      for (int k = 0; k < NV; ++k) h[k] = hv.ld2(lane, col_off<L>(64 * k, 0));
+    }
     if (c0 == 0) {
       // packed (DC, Nyquist) column: + conj(beta(u)) X(-u)* (the partner row
       // of column 0 sits in another thread: exchanged through LDS)
       __syncthreads();
 #pragma unroll
-      for (int k = 0; k < 8; ++k) buf[E::ix(tau + 64 * k, c)] = v[k];
+      for (int k = 0; k < NV; ++k) buf[E::ix(tau + 64 * k, c)] = v[k];
       __syncthreads();
       if (c == 0) {
         const float2* hb = Hbeta + (size_t)f * L;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
+        for (int k = 0; k < NV; ++k) {
           const int u = tau + 64 * k;
           const float2 pm = cconj(buf[E::ix((L - u) & (L - 1), 0)]);
           acc[k] = cadd(acc[k], cmulc(pm, hb[u]));
@@ -1272,121 +1284,13 @@ __global__ void __launch_bounds__(CT * 64) k_cols_rec3(const float2* __restrict_
       }
     }
 #pragma unroll
-    for (int k = 0; k < 8; ++k) acc[k] = cadd(acc[k], cmulc(v[k], h[k]));
+    for (int k = 0; k < NV; ++k) acc[k] = cadd(acc[k], cmulc(v[k], h[k]));
   }
   __syncthreads();
-  fft512_3<CT, +1>(acc, buf, t);
+  G::template fft<+1>(acc, buf, t);
   const BufView qv = col_view<L, CT>(Q + (size_t)b * q_stride + (size_t)g * L * NH + sp_ix<L>(0, c0));
 #pragma unroll
-  for (int k = 0; k < 8; ++k) qv.st2(acc[k], lane, col_off<L>(64 * k, 0));
-}
-
-// The same two passes at L = 1024 on the 16 x 8 x 8 engine with 128 threads
-// per column (Col3m): the filter product is formed in the engine's spectral
-// layout (rows q + 128 s), between the forward transform (natural in,
-// spectral out) and the inverse (spectral in, natural out).
-template <int CT>
-__global__ void __launch_bounds__(CT * 128) k_cols_dec3k(const float2* __restrict__ Y1, long long y1_stride,
-                                                     float2* __restrict__ Tout, long long t_stride,
-                                                     const float2* __restrict__ Hmain, const float2* __restrict__ Hbeta,
-                                                     BandMap map, const float2* __restrict__ tw) {
-  constexpr int L = 1024, NH = L / 2;
-  using E = Col3m<CT>;
-  __shared__ float2 buf[E::LDS];
-  int tile, slot, b;
-  col_block_order_lines<(16 / CT > 1 ? 16 / CT : 1)>(tile, slot, b);
-  const int p = map_u8(map.order, slot);
-  const int j = map_u8(map.scale_of, p), f = map_u8(map.filt_of, p);
-  const int c0 = tile * CT;
-  const int c = E::col(), q = E::q();
-  const float2* src = Y1 + (size_t)b * y1_stride + (size_t)j * L * NH + sp_ix<L>(0, c0);
-  const BufView xv = col_view<L, CT>(src);
-  const BufView hv = col_view<L, CT>(Hmain + (size_t)f * L * NH + sp_ix<L>(0, c0));
-  const unsigned slane = col_off<L>(q, c);
-  float2 x[8], h[8];
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    x[k] = xv.ld2(slane, col_off<L>(128 * k, 0));
-    h[k] = hv.ld2(slane, col_off<L>(128 * k, 0));
-  }
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int k = 0; k < 8; ++k) x[k] = cmul(h[k], x[k]);
-  if (c0 == 0 && c == 0) {
-    // packed (DC, Nyquist) column: + beta(u) conj(X(-u))
-    const float2* hb = Hbeta + (size_t)f * L;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const int u = q + 128 * k;
-      const float2 pm = cconj(src[sp_ix<L>((L - u) & (L - 1), 0)]);
-      x[k] = cadd(x[k], cmul(hb[u], pm));
-    }
-  }
-  fft1024_inv<CT>(x, buf, tw);
-  const BufView tv = col_view<L, CT>(Tout + (size_t)b * t_stride + (size_t)p * L * NH + sp_ix<L>(0, c0));
-  const unsigned nlane = col_off<L>(E::in_row(q), c);
-#pragma unroll
-  for (int k = 0; k < 8; ++k) tv.st2(x[k], nlane, col_off<L>(128 * k, 0));
-}
-
-template <int CT>
-__global__ void __launch_bounds__(CT * 128) k_cols_rec3k(const float2* __restrict__ U, long long u_stride,
-                                                     float2* __restrict__ Q, long long q_stride,
-                                                     const float2* __restrict__ Hmain, const float2* __restrict__ Hbeta,
-                                                     BandMap map, const float2* __restrict__ tw) {
-  constexpr int L = 1024, NH = L / 2;
-  using E = Col3m<CT>;
-  __shared__ float2 buf[E::LDS];
-  int tile, slot, b;
-  col_block_order(tile, slot, b, map.gshare);
-  const int g = map_u16(map.gorder, slot);
-  const int c0 = tile * CT;
-  const int c = E::col(), q = E::q();
-  const int p0 = map_u16(map.group_band0, g), p1 = map_u16(map.group_band0, g + 1);
-  const float2* ub = U + (size_t)b * u_stride + sp_ix<L>(0, c0);
-  const unsigned nlane = col_off<L>(E::in_row(q), c);
-  const unsigned slane = col_off<L>(q, c);
-  float2 acc[8];
-#pragma unroll
-  for (int k = 0; k < 8; ++k) acc[k] = make_float2(0.f, 0.f);
-  for (int p = p0; p < p1; ++p) {
-    const int f = map_u8(map.filt_of, p);
-    const BufView uv = col_view<L, CT>(ub + (size_t)p * L * NH);
-    const BufView hv = col_view<L, CT>(Hmain + (size_t)f * L * NH + sp_ix<L>(0, c0));
-    float2 v[8], h[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = uv.ld2(nlane, col_off<L>(128 * k, 0));
-    __builtin_amdgcn_sched_barrier(0);
-    if (p > p0) __syncthreads();  // the previous direction's reads of buf are complete
-    fft1024_fwd<CT>(v, buf, tw);
-    // the filter tile is read after the forward transform (not held across it)
-#pragma unroll
-    for (int k = 0; k < 8; ++k) h[k] = hv.ld2(slane, col_off<L>(128 * k, 0));
-    if (c0 == 0) {
-      // packed (DC, Nyquist) column: + conj(beta(u)) X(-u)*, the partner row
-      // of column 0 exchanged through LDS
-      __syncthreads();
-#pragma unroll
-      for (int k = 0; k < 8; ++k) buf[E::ix(q + 128 * k, c)] = v[k];
-      __syncthreads();
-      if (c == 0) {
-        const float2* hb = Hbeta + (size_t)f * L;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          const int u = q + 128 * k;
-          const float2 pm = cconj(buf[E::ix((L - u) & (L - 1), 0)]);
-          acc[k] = cadd(acc[k], cmulc(pm, hb[u]));
-        }
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < 8; ++k) acc[k] = cadd(acc[k], cmulc(v[k], h[k]));
-  }
-  __syncthreads();
-  fft1024_inv<CT>(acc, buf, tw);
-  const BufView qv = col_view<L, CT>(Q + (size_t)b * q_stride + (size_t)g * L * NH + sp_ix<L>(0, c0));
-#pragma unroll
-  for (int k = 0; k < 8; ++k) qv.st2(acc[k], nlane, col_off<L>(128 * k, 0));
+  for (int k = 0; k < NV; ++k) qv.st2(acc[k], lane, col_off<L>(64 * k, 0));
 }
 
 // ---------------------------------------------------------------------------
@@ -1450,27 +1354,30 @@ struct Launch {
   template <int CT>
   static hipError_t cols_dec3_ct(const float2* Y1, long long ys, float2* To, long long ts, const float2* Hm,
                                  const float2* Hb, const BandMap& map, int nimg, const float2* tw, hipStream_t s) {
-    if constexpr (L == 512 && CT >= 4)
+    if constexpr ((L == 512 && CT >= 4) || L == 1024)
       hipLaunchKernelGGL((k_cols_dec3<L, CT>), dim3(L / 2 / CT, map.nbands, nimg), dim3(CT * 64), 0, s, Y1, ys, To,
                          ts, Hm, Hb, map, tw);
-    if constexpr (L == 1024)
-      hipLaunchKernelGGL((k_cols_dec3k<CT>), dim3(L / 2 / CT, map.nbands, nimg), dim3(CT * 128), 0, s, Y1, ys, To, ts,
-                         Hm, Hb, map, tw);
     return hipGetLastError();
   }
   template <int CT>
   static hipError_t cols_rec3_ct(const float2* U, long long us, float2* Q, long long qs, const float2* Hm,
                                  const float2* Hb, const BandMap& map, int nimg, const float2* tw, hipStream_t s) {
-    if constexpr (L == 512 && CT >= 4)
+    if constexpr ((L == 512 && CT >= 4) || L == 1024)
       hipLaunchKernelGGL((k_cols_rec3<L, CT>), dim3(L / 2 / CT, map.ngroups, nimg), dim3(CT * 64), 0, s, U, us, Q, qs,
-                         Hm, Hb, map, tw);
-    if constexpr (L == 1024)
-      hipLaunchKernelGGL((k_cols_rec3k<CT>), dim3(L / 2 / CT, map.ngroups, nimg), dim3(CT * 128), 0, s, U, us, Q, qs,
                          Hm, Hb, map, tw);
     return hipGetLastError();
   }
-  // ct: column tile width (8 or 16; 0 = default for L); -4 / -8: the
-  // three-pass engine with 4 / 8 columns (L = 512 and 1024, pre only)
+  // ct: column tile width (4, 8 or 16; 0 = the default below); -2 / -4 / -8: the
+  // engines with 64 threads per column with 2 / 4 / 8 columns (L = 512 and
+  // 1024, pre only).  Defaults, by timing whole denoise steps with every tile:
+  // the narrowest tile runs the most blocks (a quarter of the 16-column tile's
+  // time is a half-empty chip for one image: 256^2 reconstruction 17 -> 12 us)
+  // and since spectra are stored in strips it costs no bandwidth.  The
+  // reconstruction at 512 and 1024 takes the 64-thread engine (512^2 step
+  // 129 -> 116 us against 117 with 4 two-pass columns; 4 x 1024^2, groups of 8,
+  // 1188 -> 1165 us), for one 1024^2 image with 2 columns (381 -> 375 us);
+  // the decomposition does not (1024^2: 392 against 420 us).
+  static constexpr int kDefaultTile = ColTile<L>::narrow ? 4 : (ColTile<L>::dflt < 8 ? ColTile<L>::dflt : 8);
   static hipError_t cols_dec(const float2* Y1, long long ys, float2* To, long long ts, const float2* Hm,
                              const float2* Hb, const BandMap& map, int nimg, const float2* tw, hipStream_t s, int ct,
                              bool pre) {
@@ -1481,7 +1388,7 @@ struct Launch {
       if (ct == -8) return cols_dec3_ct<8>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s);
       return hipErrorInvalidValue;
     }
-    if (ct == 0) ct = ColTile<L>::dflt;
+    if (ct == 0) ct = kDefaultTile;
     if (ct == 4 && ColTile<L>::narrow)
       return cols_dec_ct<(ColTile<L>::narrow ? 4 : 8)>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, pre);
     if (ct == 8) return cols_dec_ct<8>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, pre);
@@ -1490,7 +1397,7 @@ struct Launch {
     return hipErrorInvalidValue;
   }
   static hipError_t cols_fwd(float2* Y1, long long ys, int nplanes, int nimg, const float2* tw, hipStream_t s, int ct) {
-    if (ct <= 0) ct = ColTile<L>::dflt;
+    if (ct <= 0) ct = kDefaultTile;
     if (ct == 4 && ColTile<L>::narrow) return cols_fwd_ct<(ColTile<L>::narrow ? 4 : 8)>(Y1, ys, nplanes, nimg, tw, s);
     if (ct == 8) return cols_fwd_ct<8>(Y1, ys, nplanes, nimg, tw, s);
     if (ct == 16 && ColTile<L>::wide) return cols_fwd_ct<(ColTile<L>::wide ? 16 : 8)>(Y1, ys, nplanes, nimg, tw, s);
@@ -1498,6 +1405,7 @@ struct Launch {
   }
   static hipError_t cols_rec(const float2* U, long long us, float2* Q, long long qs, const float2* Hm,
                              const float2* Hb, const BandMap& map, int nimg, const float2* tw, hipStream_t s, int ct) {
+    if (ct == 0) ct = L == 1024 ? (nimg == 1 ? -2 : -4) : (L == 512 ? -4 : kDefaultTile);
     if (ct < 0) {
       if (L != 512 && L != 1024) return hipErrorInvalidValue;
       if (ct == -2 && L == 1024) return cols_rec3_ct<2>(U, us, Q, qs, Hm, Hb, map, nimg, tw, s);
@@ -1505,7 +1413,6 @@ struct Launch {
       if (ct == -8) return cols_rec3_ct<8>(U, us, Q, qs, Hm, Hb, map, nimg, tw, s);
       return hipErrorInvalidValue;
     }
-    if (ct == 0) ct = ColTile<L>::dflt;
     if (ct == 4 && ColTile<L>::narrow) return cols_rec_ct<(ColTile<L>::narrow ? 4 : 8)>(U, us, Q, qs, Hm, Hb, map, nimg, tw, s);
     if (ct == 8) return cols_rec_ct<8>(U, us, Q, qs, Hm, Hb, map, nimg, tw, s);
     if (ct == 16 && ColTile<L>::wide) return cols_rec_ct<(ColTile<L>::wide ? 16 : 8)>(U, us, Q, qs, Hm, Hb, map, nimg, tw, s);
