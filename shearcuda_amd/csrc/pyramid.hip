@@ -359,15 +359,45 @@ struct PyrCfg<2> {
   static constexpr int TH = 32, TW = 64, VS = 8, HS = 8, T = 256;
 };
 
-template <int P, bool ADJ, int V>
-static hipError_t one2two_v(const float* x, float* ya, float* yb, const ImgStrides& st, int nimg, int L, int m,
+// Variant 0 where its 16 x 32 tiles would leave CUs idle (fewer than 256 blocks: one
+// image of up to 256^2): a quarter of the tile, fewer values per thread.  Same
+// sums in the same order.  Decomposition + reconstruction of one image: 64^2 66 ->
+// 59 us, 128^2 75 -> 68 us, 256^2 97 -> 93 us; at 512^2 (512 blocks) no gain.
+struct PyrSmall {
+  static constexpr int TH = 8, TW = 16, VS = 2, HS = 1, T = 256;
+};
+constexpr long long PYR_SMALL_TILES = 256;
+static long long tiles_of(int nout, int th, int tw, int m, int nimg) {
+  return (long long)((nout + th - 1) / th) * ((nout + tw - 1) / tw) * m * m * nimg;
+}
+
+template <int P, bool ADJ, class C>
+static hipError_t one2two_c(const float* x, float* ya, float* yb, const ImgStrides& st, int nimg, int L, int m,
                             hipStream_t s) {
-  using C = PyrCfg<V>;
   const int nout = (ADJ ? L + 2 * HALO * m : L) / m;
   dim3 grid((nout + C::TW - 1) / C::TW, (nout + C::TH - 1) / C::TH, m * m * nimg);
   hipLaunchKernelGGL((k_pyr_one2two<P, ADJ, C::TH, C::TW, C::VS, C::HS, C::T>), grid, dim3(C::T), 0, s, x, ya,
                      yb, st, L, m);
   return hipGetLastError();
+}
+template <int P, bool ADJ, class C>
+static hipError_t two2one_c(const float* xa, const float* xb, float* out, const ImgStrides& st, int nimg, int L,
+                            int m, const LowThresh& lt, float sa, float sb, hipStream_t s) {
+  const int nout = (ADJ ? L + 2 * HALO * m : L) / m;
+  dim3 grid((nout + C::TW - 1) / C::TW, (nout + C::TH - 1) / C::TH, m * m * nimg);
+  hipLaunchKernelGGL((k_pyr_two2one<P, ADJ, C::TH, C::TW, C::VS, C::HS, C::T>), grid, dim3(C::T), 0, s, xa, xb,
+                     out, st, L, m, lt, sa, sb);
+  return hipGetLastError();
+}
+
+template <int P, bool ADJ, int V>
+static hipError_t one2two_v(const float* x, float* ya, float* yb, const ImgStrides& st, int nimg, int L, int m,
+                            hipStream_t s) {
+  using C = PyrCfg<V>;
+  const int nout = (ADJ ? L + 2 * HALO * m : L) / m;
+  if (V == 0 && tiles_of(nout, C::TH, C::TW, m, nimg) < PYR_SMALL_TILES)
+    return one2two_c<P, ADJ, PyrSmall>(x, ya, yb, st, nimg, L, m, s);
+  return one2two_c<P, ADJ, C>(x, ya, yb, st, nimg, L, m, s);
 }
 
 template <int P, bool ADJ, int V>
@@ -375,10 +405,9 @@ static hipError_t two2one_v(const float* xa, const float* xb, float* out, const 
                             int m, const LowThresh& lt, float sa, float sb, hipStream_t s) {
   using C = PyrCfg<V>;
   const int nout = (ADJ ? L + 2 * HALO * m : L) / m;
-  dim3 grid((nout + C::TW - 1) / C::TW, (nout + C::TH - 1) / C::TH, m * m * nimg);
-  hipLaunchKernelGGL((k_pyr_two2one<P, ADJ, C::TH, C::TW, C::VS, C::HS, C::T>), grid, dim3(C::T), 0, s, xa, xb,
-                     out, st, L, m, lt, sa, sb);
-  return hipGetLastError();
+  if (V == 0 && tiles_of(nout, C::TH, C::TW, m, nimg) < PYR_SMALL_TILES)
+    return two2one_c<P, ADJ, PyrSmall>(xa, xb, out, st, nimg, L, m, lt, sa, sb, s);
+  return two2one_c<P, ADJ, C>(xa, xb, out, st, nimg, L, m, lt, sa, sb, s);
 }
 
 static bool level_ok(int L, int m, int nimg) { return m >= 1 && L % m == 0 && nimg >= 1 && m * m * nimg <= 65535; }
