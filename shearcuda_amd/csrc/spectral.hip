@@ -120,6 +120,24 @@ __device__ __forceinline__ float2 shfl2(float2 v, int src) {
   return make_float2(__shfl(v.x, src), __shfl(v.y, src));
 }
 
+// Band spectra are accessed non-temporally where one image's exceed the L2s (from
+// 512^2 on: 50 MB).  At 256^2 (12.6 MB) only the column passes' stores are, and
+// only in batches (48 x 256^2: 922 -> 875 us of kernels; one image, whose next
+// kernel reads them from the L2s: 84 us for the transform pair, non-temporal 86);
+// choosing the loads there at run time too broke up their batches (870 us a step
+// against 800).
+template <int L>
+__device__ __forceinline__ float2 band_ld(const float2* p) {
+  return L >= 512 ? load_nt(p) : *p;
+}
+template <int L>
+__device__ __forceinline__ void band_st(float2* p, float2 v) {
+  if constexpr (L >= 512)
+    store_nt(p, v);
+  else
+    *p = v;
+}
+
 template <int E, int PADSH>
 constexpr int lds_size() {
   return E + (E >> PADSH) + 1;
@@ -211,7 +229,7 @@ __device__ __forceinline__ void row_fwd_from_A(float2 (&v)[R2], bool validA, int
     const float2 zm = (k2 == 0) ? u[(R1 - k1) & (R1 - 1)] : sh;
     const float2 val = (k == 0) ? make_float2(u[0].x + u[0].y, u[0].x - u[0].y)
                                 : r2c_post(u[k1], zm, ctw_mul<L / R2, -1>(t.w0, k1));
-    if (validB) drow[(size_t)(R2 * k1) * L] = val;
+    if (validB) band_st<L>(drow + (size_t)(R2 * k1) * L, val);
   }
 }
 
@@ -252,7 +270,7 @@ __device__ __forceinline__ void gather_row(const float2* __restrict__ row, int n
                                            float2 (&xm)[R2]) {
   static_assert(64 % R1 == 0, "a row's lanes lie in one wave");
 #pragma unroll
-  for (int n2 = 0; n2 < R2; ++n2) x[n2] = row[sp_ix<2 * N>(0, n1) + (size_t)(R1 * n2) * 2 * N];
+  for (int n2 = 0; n2 < R2; ++n2) x[n2] = band_ld<2 * N>(row + sp_ix<2 * N>(0, n1) + (size_t)(R1 * n2) * 2 * N);
   const int lane = threadIdx.x & 63;
   const int src = (lane & ~(R1 - 1)) | ((R1 - n1) & (R1 - 1));
 #pragma unroll
@@ -385,7 +403,7 @@ __device__ __forceinline__ void row_inv_to_B_lds(float2 (&u)[R1], bool validA, i
 template <int N, int R1, int R2>
 __device__ __forceinline__ void load_row_x(const float2* __restrict__ row, int n1, float2 (&x)[R2]) {
 #pragma unroll
-  for (int n2 = 0; n2 < R2; ++n2) x[n2] = row[sp_ix<2 * N>(0, n1) + (size_t)(R1 * n2) * 2 * N];
+  for (int n2 = 0; n2 < R2; ++n2) x[n2] = band_ld<2 * N>(row + sp_ix<2 * N>(0, n1) + (size_t)(R1 * n2) * 2 * N);
 }
 
 // Row real-to-complex FFT (packed output), optional hard threshold on load.
@@ -519,7 +537,7 @@ __global__ void __launch_bounds__(RowCfg<L>::T) k_rows_c2r_r2c(PlaneSet Tin, Pla
 #pragma unroll
     for (int k1 = 0; k1 < R1; ++k1) {
       const float2 c = u[k1];
-      if (store_c) cdst[(size_t)rB * N + k2 + R2 * k1] = c;
+      if (store_c) band_st<L>(cdst + (size_t)rB * N + k2 + R2 * k1, c);
       u[k1] = shrink2(c, t, rule);
     }
     __syncthreads();  // pass-B reads of buf are complete
@@ -578,7 +596,7 @@ __global__ void __launch_bounds__(RowCfg<L>::T) k_rows_c2r_mask_r2c(PlaneSet Tin
   // during the inverse transform
   float2 cv[R1];
 #pragma unroll
-  for (int k1 = 0; k1 < R1; ++k1) cv[k1] = csrc[(size_t)rB * N + k2 + R2 * k1];
+  for (int k1 = 0; k1 < R1; ++k1) cv[k1] = band_ld<L>(csrc + (size_t)rB * N + k2 + R2 * k1);
   float2 u[R1];
   if constexpr (L >= 1024) {
     auto gather = [&](int rr, int nn, float2 (&x)[R2]) { load_row_x<N, R1, R2>(src + sp_ix<L>(rr, 0), nn, x); };
@@ -672,7 +690,8 @@ __device__ __forceinline__ void col_load_A(float2 (&v)[Split<L>::R2], const floa
   const BufView bv = col_view<L, CT>(src);
   const unsigned lane = col_off<L>(threadIdx.x / CT, threadIdx.x % CT);
 #pragma unroll
-  for (int n2 = 0; n2 < R2; ++n2) v[n2] = bv.ld2(lane, col_off<L>(R1 * n2, 0));
+  for (int n2 = 0; n2 < R2; ++n2)
+    v[n2] = L >= 512 ? bv.ld2nt(lane, col_off<L>(R1 * n2, 0)) : bv.ld2(lane, col_off<L>(R1 * n2, 0));
 }
 
 // Pass-B registers of thread (c, k2): x[k1] = src(k2 + R2 k1, c).
@@ -712,8 +731,10 @@ __device__ __forceinline__ void col_fwd_A(const float2* __restrict__ src, float2
     float2 v[R1];
     const BufView bv = col_view<L, CT>(src);
     const unsigned lane = col_off<L>(n1 + R1 * h, c);
+    // (this form: L = 512 and the small sizes)
 #pragma unroll
-    for (int j = 0; j < R1; ++j) v[j] = bv.ld2(lane, col_off<L>(2 * R1 * j, 0));
+    for (int j = 0; j < R1; ++j)
+      v[j] = L >= 512 ? bv.ld2nt(lane, col_off<L>(2 * R1 * j, 0)) : bv.ld2(lane, col_off<L>(2 * R1 * j, 0));
     PairTw<R1> t;
     pair_tw<R1, 1>(t, n1, h, tw);
     __builtin_amdgcn_sched_barrier(0);  // data and twiddle loads in flight together
@@ -886,7 +907,12 @@ __device__ __forceinline__ void col_inv_from_B(float2 (&q)[Split<L>::R1], float2
     const BufView bv = col_view<L, CT>(dst);
     const unsigned lane = col_off<L>(kb + R1 * R1 * h, cp);
 #pragma unroll
-    for (int k = 0; k < R1; ++k) bv.st2(w[k], lane, col_off<L>(R1 * k, 0));
+    for (int k = 0; k < R1; ++k) {
+      if constexpr (L >= 512)
+        bv.st2nt(w[k], lane, col_off<L>(R1 * k, 0));
+      else
+        bv.st2(w[k], lane, col_off<L>(R1 * k, 0));
+    }
     return;
   }
   const int kb = tid / CT;
@@ -898,8 +924,13 @@ __device__ __forceinline__ void col_inv_from_B(float2 (&q)[Split<L>::R1], float2
     dft<R2, +1>(w);
     const BufView bv = col_view<L, CT>(dst);
     const unsigned lane = col_off<L>(kb, c);
+    if (L >= 512 || (L == 256 && gridDim.z > 1)) {
 #pragma unroll
-    for (int k1 = 0; k1 < R2; ++k1) bv.st2(w[k1], lane, col_off<L>(R1 * k1, 0));
+      for (int k1 = 0; k1 < R2; ++k1) bv.st2nt(w[k1], lane, col_off<L>(R1 * k1, 0));
+    } else {
+#pragma unroll
+      for (int k1 = 0; k1 < R2; ++k1) bv.st2(w[k1], lane, col_off<L>(R1 * k1, 0));
+    }
   }
 }
 
@@ -1201,7 +1232,7 @@ __global__ void __launch_bounds__(CT * 64) k_cols_dec3(const float2* __restrict_
   G::template fft<+1>(q, buf, t);
   const BufView tv = col_view<L, CT>(Tout + (size_t)b * t_stride + (size_t)p * L * NH + sp_ix<L>(0, c0));
 #pragma unroll
-  for (int k = 0; k < NV; ++k) tv.st2(q[k], lane, col_off<L>(64 * k, 0));
+  for (int k = 0; k < NV; ++k) tv.st2nt(q[k], lane, col_off<L>(64 * k, 0));
 }
 
 template <int L, int CT>
@@ -1236,7 +1267,7 @@ __global__ void __launch_bounds__(CT * 64) k_cols_rec3(const float2* __restrict_
   if constexpr (ahead) {
     const BufView uv = col_view<L, CT>(ub + (size_t)p0 * L * NH);
 #pragma unroll
-    for (int k = 0; k < NV; ++k) vn[k] = uv.ld2(lane, col_off<L>(64 * k, 0));
+    for (int k = 0; k < NV; ++k) vn[k] = uv.ld2nt(lane, col_off<L>(64 * k, 0));
   }
   for (int p = p0; p < p1; ++p) {
     const int f = map_u8(map.filt_of, p);
@@ -1252,12 +1283,12 @@ __global__ void __launch_bounds__(CT * 64) k_cols_rec3(const float2* __restrict_
     if constexpr (!ahead) {
       const BufView uv = col_view<L, CT>(ub + (size_t)p * L * NH);
 #pragma unroll
-      for (int k = 0; k < NV; ++k) v[k] = uv.ld2(lane, col_off<L>(64 * k, 0));
+      for (int k = 0; k < NV; ++k) v[k] = uv.ld2nt(lane, col_off<L>(64 * k, 0));
     }
     if (ahead && p + 1 < p1) {
       const BufView uv = col_view<L, CT>(ub + (size_t)(p + 1) * L * NH);
 #pragma unroll
-      for (int k = 0; k < NV; ++k) vn[k] = uv.ld2(lane, col_off<L>(64 * k, 0));
+      for (int k = 0; k < NV; ++k) vn[k] = uv.ld2nt(lane, col_off<L>(64 * k, 0));
     }
     __builtin_amdgcn_sched_barrier(0);
     if (p > p0) __syncthreads();  // the previous direction's reads of buf are complete
