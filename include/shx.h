@@ -293,6 +293,21 @@ int shx_mrdwt_adjoint(const float* yl_bar, const float* yh_bar, int m, int n, co
 int shx_mirdwt_adjoint(const float* x_bar, int m, int n, const double* h, int lh, int L, float* yl_bar,
                        float* yh_bar, float* work, int nimg, void* stream);
 
+/* Soft-thresholded synthesis and its backward, with the thresholds applied inside
+ * the level kernels; available where shx_rdwt_fused(n, L, lh) is 1 (filters of at
+ * most 8 taps, rows of at most 512 or dilated filters of at most 256 columns).
+ * th_dev: 1 + 3 L thresholds (yl, then [lh hl hh] per level), shared by the images.
+ * shx_mirdwt_soft: x = mirdwt(soft(yl), soft(yh)); work: 2*m*n*nimg floats.
+ * shx_wave_shrink_mask: with (c_l, c_h) = mrdwt(b) and the output gradient g,
+ * gyl, gyh = mirdwt^T(g) where |c| > th, else 0, and gth_dev (not cleared) +=
+ * sum -sign(c) 1[|c| > th] mirdwt^T(g) per band; work: 4*m*n*nimg floats. */
+int shx_rdwt_fused(int n, int L, int lh);
+int shx_mirdwt_soft(const float* yl, const float* yh, int m, int n, const double* h, int lh, int L,
+                    const float* th_dev, float* x, float* work, int nimg, void* stream);
+int shx_wave_shrink_mask(const float* b, const float* g, int m, int n, const double* h, int lh, int L,
+                         const float* th_dev, float* gyl, float* gyh, float* gth_dev, float* work, int nimg,
+                         void* stream);
+
 /* Soft threshold with one threshold per band (th_dev, device FP32) over a
  * batched layout: element e of each image (img_elems elements) belongs to
  * band band_off + ((e mod rowlen) / seglen).  NSST stacks: rowlen =

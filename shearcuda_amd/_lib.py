@@ -81,6 +81,11 @@ _SIGNATURES = [
                                   c_int, c_void_p]),
     ("shx_mirdwt_adjoint", c_int, [c_void_p, c_int, c_int, P(c_double), c_int, c_int, c_void_p, c_void_p, c_void_p,
                                    c_int, c_void_p]),
+    ("shx_rdwt_fused", c_int, [c_int, c_int, c_int]),
+    ("shx_mirdwt_soft", c_int, [c_void_p, c_void_p, c_int, c_int, P(c_double), c_int, c_int, c_void_p, c_void_p,
+                                c_void_p, c_int, c_void_p]),
+    ("shx_wave_shrink_mask", c_int, [c_void_p, c_void_p, c_int, c_int, P(c_double), c_int, c_int, c_void_p, c_void_p,
+                                     c_void_p, c_void_p, c_void_p, c_int, c_void_p]),
     ("shx_soft_bands", c_int, [c_void_p, c_void_p, c_int, c_int64, c_int64, c_int64, c_int, c_void_p, c_void_p]),
     ("shx_soft_bands_backward", c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int64, c_int64,
                                         c_int, c_void_p, c_void_p]),

@@ -2278,6 +2278,29 @@ int shx_mirdwt_adjoint(const float* x_bar, int m, int n, const double* h, int lh
                   [&](float* t) { return shx::rdwt_analysis(x_bar, yl_bar, yh_bar, t, m, n, L, f, nimg, s); });
 }
 
+int shx_rdwt_fused(int n, int L, int lh) { return shx::rdwt_fused(n, L, lh) ? 1 : 0; }
+
+int shx_mirdwt_soft(const float* yl, const float* yh, int m, int n, const double* h, int lh, int L,
+                    const float* th_dev, float* x, float* work, int nimg, void* stream) {
+  if (int r = rdwt_check(m, n, h, lh, L, nimg)) return r;
+  if (!x || !yl || !yh || !th_dev || !work) return fail(SHX_ERR_ARG, "null input, thresholds, output or workspace");
+  if (!shx::rdwt_fused(n, L, lh)) return fail(SHX_ERR_UNSUPPORTED, "no fused levels for rows of %d, %d levels, %d taps", n, L, lh);
+  SHX_HIP(shx::rdwt_synthesis(yl, yh, x, work, m, n, L, rdwt_taps(h, lh, true, 1.0), nimg, (hipStream_t)stream, th_dev));
+  return SHX_OK;
+}
+
+int shx_wave_shrink_mask(const float* b, const float* g, int m, int n, const double* h, int lh, int L,
+                         const float* th_dev, float* gyl, float* gyh, float* gth_dev, float* work, int nimg,
+                         void* stream) {
+  if (int r = rdwt_check(m, n, h, lh, L, nimg)) return r;
+  if (!b || !g || !th_dev || !gyl || !gyh || !gth_dev || !work)
+    return fail(SHX_ERR_ARG, "null input, thresholds, output or workspace");
+  if (!shx::rdwt_fused(n, L, lh)) return fail(SHX_ERR_UNSUPPORTED, "no fused levels for rows of %d, %d levels, %d taps", n, L, lh);
+  SHX_HIP(shx::rdwt_shrink_mask(b, g, gyl, gyh, work, m, n, L, rdwt_taps(h, lh, false, 1.0), th_dev, gth_dev, nimg,
+                                (hipStream_t)stream));
+  return SHX_OK;
+}
+
 int shx_norm_pow(const float* x, int64_t n, double p, double* out, void* stream) {
   if (!x || !out) return fail(SHX_ERR_ARG, "null input or output");
   hipStream_t s = (hipStream_t)stream;

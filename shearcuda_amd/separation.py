@@ -126,9 +126,18 @@ class WaveShrink(torch.autograd.Function):
         b = b.contiguous()
         B, m, n = b.shape
         yl, yh = api.mrdwt_cuda(b, h, levels)
-        yls = soft_bands(yl, th, B, m * n, m * n, m * n, 0)
-        yhs = soft_bands(yh, th, B, m * 3 * n * levels, 3 * n * levels, n, 1)
-        out = api.mirdwt_cuda(yls, yhs, h, levels)
+        _check_layout(yl, th, B, m * n, m * n, m * n, 0)
+        _check_layout(yh, th, B, m * 3 * n * levels, 3 * n * levels, n, 1)
+        hv, hp = api._h_arg(h)
+        if lib.shx_rdwt_fused(n, int(levels), hv.size):
+            out = torch.empty_like(b)
+            work = api._workspace(2 * b.numel(), b.device)
+            check(lib.shx_mirdwt_soft(_vp(yl), _vp(yh), m, n, hp, hv.size, int(levels), _vp(th), _vp(out), _vp(work),
+                                      B, _stream()))
+        else:
+            yls = soft_bands(yl, th, B, m * n, m * n, m * n, 0)
+            yhs = soft_bands(yh, th, B, m * 3 * n * levels, 3 * n * levels, n, 1)
+            out = api.mirdwt_cuda(yls, yhs, h, levels)
         ctx.save_for_backward(b, th)
         ctx.h, ctx.levels = h, levels
         return out
@@ -138,9 +147,20 @@ class WaveShrink(torch.autograd.Function):
         b, th = ctx.saved_tensors
         h, levels = ctx.h, ctx.levels
         B, m, n = b.shape
+        gth = torch.zeros_like(th)
+        hv, hp = api._h_arg(h)
+        if lib.shx_rdwt_fused(n, int(levels), hv.size):
+            # the forward's bands are recomputed inside the level kernels
+            g = g.contiguous()
+            api._require_shape(g, b.shape, "gradient")
+            gyl = torch.empty_like(b)
+            gyh = torch.empty(b.shape[:-1] + (3 * n * levels,), device=b.device, dtype=torch.float32)
+            work = api._workspace(4 * b.numel(), b.device)
+            check(lib.shx_wave_shrink_mask(_vp(b), _vp(g), m, n, hp, hv.size, int(levels), _vp(th), _vp(gyl),
+                                           _vp(gyh), _vp(gth), _vp(work), B, _stream()))
+            return api.mrdwt_adjoint_cuda(gyl, gyh, h, levels), gth, None, None
         yl, yh = api.mrdwt_cuda(b, h, levels)       # recomputed bands
         gyl, gyh = api.mirdwt_adjoint_cuda(g.contiguous(), h, levels)
-        gth = torch.zeros_like(th)
         gyl = soft_bands_backward(yl, gyl, th, gth, B, m * n, m * n, m * n, 0)
         gyh = soft_bands_backward(yh, gyh, th, gth, B, m * 3 * n * levels, 3 * n * levels, n, 1)
         gb = api.mrdwt_adjoint_cuda(gyl, gyh, h, levels)

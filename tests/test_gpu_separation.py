@@ -125,3 +125,34 @@ def test_hard_bands_forward_backward(gpu):
     keep = x.abs() > t
     assert torch.equal(y, torch.where(keep, x, torch.zeros_like(x)))
     assert torch.equal(gx, torch.where(keep, gy, torch.zeros_like(gy)))
+
+
+@pytest.mark.parametrize("shape,levels,name", [((2, 8, 8), 3, "Haar"), ((1, 36, 1044), 2, "Daubechies"),
+                                               ((3, 64, 512), 3, "Daubechies"), ((1, 144, 96), 4, "Symmlet")])
+def test_fused_wave_shrink_equals_separate_calls(gpu, shape, levels, name):
+    """Soft thresholds inside the wavelet level kernels against the separate
+    transform, threshold and transpose calls: outputs and input gradients to
+    FP32 rounding of the transform, threshold gradients to that of a sum over
+    a band."""
+    from shearcuda_amd import api, separation
+    from shearcuda_amd.wavelets import MakeONFilter
+    h = MakeONFilter(name, 4)
+    B, m, n = shape
+    rng = np.random.default_rng(sum(shape))
+    b = torch.tensor(rng.standard_normal(shape) * 20, dtype=torch.float32, device="cuda")
+    g = torch.tensor(rng.standard_normal(shape), dtype=torch.float32, device="cuda")
+    th = torch.tensor(rng.uniform(2.0, 15.0, 1 + 3 * levels), dtype=torch.float32, device="cuda")
+    bb, tt = b.clone().requires_grad_(True), th.clone().requires_grad_(True)
+    out = separation.WaveShrink.apply(bb, tt, h, levels)
+    gb, gt = torch.autograd.grad(out, [bb, tt], g)
+    yl, yh = api.mrdwt_cuda(b, h, levels)
+    lay = [(B, m * n, m * n, m * n, 0), (B, m * 3 * n * levels, 3 * n * levels, n, 1)]
+    want = api.mirdwt_cuda(separation.soft_bands(yl, th, *lay[0]), separation.soft_bands(yh, th, *lay[1]), h, levels)
+    gyl, gyh = api.mirdwt_adjoint_cuda(g, h, levels)
+    gth = torch.zeros_like(th)
+    gyl = separation.soft_bands_backward(yl, gyl, th, gth, *lay[0])
+    gyh = separation.soft_bands_backward(yh, gyh, th, gth, *lay[1])
+    gw = api.mrdwt_adjoint_cuda(gyl, gyh, h, levels)
+    assert torch.equal(out.detach(), want)
+    assert torch.equal(gb, gw)
+    assert float((gt - gth).abs().max()) <= 1e-5 * float(g.abs().sum())
