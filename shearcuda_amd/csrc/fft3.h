@@ -92,111 +92,6 @@ __device__ __forceinline__ void fft512_3(float2 (&v)[8], float2* buf, const Fft3
   dft8<DIR>(v);
 }
 
-// ---- 1024 points = 16 x 8 x 8 on 128 threads per column ---------------------
-// Thread tid of CT * 128 threads: column c = (tid / 2) % CT and column-local
-// index q = (tid & 1) + 2 (tid / (2 CT)) in [0, 128), so that the two halves
-// of each radix-16 DFT of stage 1 sit in adjacent lanes (dft_pair).  With
-// n = a + 64 b (a < 64, b < 16) and k = p + 16 q' (p < 16, q' < 64):
-//   stage 1 (a = q / 2, lane half h = q & 1, holding b = 2 j + h, j < 8):
-//                         Z_p[a] = w1024^(a p) DFT16_b x[a + 64 b], p = k + 8 h
-//   stage 2 (p = q & 15, a0 = q / 16):
-//                         V_{p,a0}[r] = w64^(a0 r) DFT8_a1 Z_p[a0 + 8 a1]
-//   stage 3 (p = q & 15, r = q / 16):
-//                         X[p + 16 r + 128 s] = DFT8_a0 V_{p,a0}[r] = X[q + 128 s]
-// The forward transform takes the "natural" layout v[j] = x[in_row(q) +
-// 128 j], in_row(q) = q / 2 + 64 (q & 1), and returns the spectral layout
-// v[s] = X[q + 128 s].  The inverse runs the conjugated stages in reverse
-// order (spectral in, natural out; both unnormalised).
-template <int CT>
-struct Col3m {
-  static constexpr int N = 1024, TPC = 128, T = CT * TPC;
-  // one pad of CT after every 64 rows and, for CT >= 4, 16 more after row
-  // 511 (the stage-1 stores of a lane pair are 512 rows apart)
-  static constexpr int PADH = CT >= 4 ? 16 : 0;
-  static constexpr int LDS = N * CT + (N / 64) * CT + PADH;
-  __device__ static __forceinline__ int ix(int e, int c) { return e * CT + c + (e >> 6) * CT + (e >> 9) * PADH; }
-  __device__ static __forceinline__ int col() { return (threadIdx.x >> 1) % CT; }
-  __device__ static __forceinline__ int q() { return (threadIdx.x & 1) + 2 * (threadIdx.x / (2 * CT)); }
-  __device__ static __forceinline__ int in_row(int q) { return (q >> 1) + 64 * (q & 1); }
-};
-
-// Transpose of dft_pair: the thread holds X[k + R h] (k < R) and gets
-// z[j] = x[2 j + h] of the length-2R DFT with sign DIR:
-//   h = 0: DFT_R(X[k] + X[k + R]);  h = 1: DFT_R(W^k (X[k] - X[k + R])), W = w_2R^DIR.
-template <int R, int DIR>
-__device__ __forceinline__ void dft_pair_t(float2 (&z)[R], int h) {
-#pragma unroll
-  for (int k = 0; k < R; ++k) {
-    const float2 o = swap_pair(z[k]);
-    z[k] = h ? ctw_mul<2 * R, DIR>(csub(o, z[k]), k) : cadd(z[k], o);
-  }
-  dft<R, DIR>(z);
-}
-
-template <int CT>
-__device__ __forceinline__ void fft1024_fwd(float2 (&v)[8], float2* buf, const float2* __restrict__ tw_table) {
-  using E = Col3m<CT>;
-  const TwView tw(tw_table, 1024);
-  const int c = E::col(), q = E::q();
-  const int t = q >> 1, hh = q & 1, p = q & 15, a0 = q >> 4;
-  float2 w1[8], w2[8];
-#pragma unroll
-  for (int k = 0; k < 8; ++k) w1[k] = tw[t * (k + 8 * hh)];
-#pragma unroll
-  for (int r = 1; r < 8; ++r) w2[r] = tw[16 * a0 * r];
-  // stage 1: radix 16 over the lane pair
-  dft_pair<8, -1>(v, hh);
-#pragma unroll
-  for (int k = 0; k < 8; ++k) buf[E::ix((k + 8 * hh) * 64 + t, c)] = cmul(v[k], w1[k]);
-  __syncthreads();
-  // stage 2
-#pragma unroll
-  for (int a1 = 0; a1 < 8; ++a1) v[a1] = buf[E::ix(p * 64 + a0 + 8 * a1, c)];
-  dft8<-1>(v);
-#pragma unroll
-  for (int r = 1; r < 8; ++r) v[r] = cmul(v[r], w2[r]);
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < 8; ++r) buf[E::ix(p * 64 + 8 * r + a0, c)] = v[r];
-  __syncthreads();
-  // stage 3 (r = q / 16 = a0)
-#pragma unroll
-  for (int k = 0; k < 8; ++k) v[k] = buf[E::ix(p * 64 + 8 * a0 + k, c)];
-  dft8<-1>(v);
-}
-
-template <int CT>
-__device__ __forceinline__ void fft1024_inv(float2 (&v)[8], float2* buf, const float2* __restrict__ tw_table) {
-  using E = Col3m<CT>;
-  const TwView tw(tw_table, 1024);
-  const int c = E::col(), q = E::q();
-  const int t = q >> 1, hh = q & 1, p = q & 15, a0 = q >> 4;
-  float2 w1[8], w2[8];
-#pragma unroll
-  for (int k = 0; k < 8; ++k) w1[k] = tw[t * (k + 8 * hh)];
-#pragma unroll
-  for (int r = 1; r < 8; ++r) w2[r] = tw[16 * a0 * r];
-  // stage 3, conjugated (over s; r = q / 16)
-  dft8<+1>(v);
-#pragma unroll
-  for (int k = 0; k < 8; ++k) buf[E::ix(p * 64 + 8 * a0 + k, c)] = v[k];
-  __syncthreads();
-  // stage 2, conjugated: twiddles, then the DFT over r
-#pragma unroll
-  for (int r = 0; r < 8; ++r) v[r] = buf[E::ix(p * 64 + 8 * r + a0, c)];
-#pragma unroll
-  for (int r = 1; r < 8; ++r) v[r] = cmulc(v[r], w2[r]);
-  dft8<+1>(v);
-  __syncthreads();
-#pragma unroll
-  for (int a1 = 0; a1 < 8; ++a1) buf[E::ix(p * 64 + a0 + 8 * a1, c)] = v[a1];
-  __syncthreads();
-  // stage 1, conjugated: twiddles, then the transposed pair DFT
-#pragma unroll
-  for (int k = 0; k < 8; ++k) v[k] = cmulc(buf[E::ix((k + 8 * hh) * 64 + t, c)], w1[k]);
-  dft_pair_t<8, +1>(v, hh);
-}
-
 // ---- 1024 points = 16 x 8 x 8 on 64 threads per column (16 values each) ----
 // Thread (c, tau) of a block of CT * 64 threads, c = threadIdx.x % CT, holds
 // v[t] = x[tau + 64 t], t < 16, and gets X[tau + 64 t] back (same layout).

@@ -296,3 +296,30 @@ def test_slab_band_loop_equals_bands(mods, n, group, dirs, mode):
         assert err < TOL, (l, err)
     plan.close()
     sh.close()
+
+
+@pytest.mark.parametrize("n,dirs,mode,group", [(32, (3, 2, 2), 1, 1), (48, (3, 2, 2), 1.5, 3), (64, (3, 2, 2), 2, 5),
+                                               (128, (2, 2, 2), 1, 6)])
+def test_analysis_adjoint_at_ragged_groups(mods, n, dirs, mode, group):
+    """The adjoint sums a group's bands in four chunks: groups that leave
+    chunks empty or uneven, on every FFT grid, against the adjoint identity
+    and the group of 8.  The groups only reorder a sum of FP32 products, so
+    both share the identity's tolerance."""
+    print("case adjoint groups n=%d group=%d" % (n, group), flush=True)
+    sh = mods[1].Shear3D(n, dirs, mode)
+    rng = np.random.default_rng(n + group)
+    s = torch.tensor(rng.standard_normal((1, sh.subs_elems)), dtype=torch.float32, device="cuda")
+    y = torch.tensor(rng.standard_normal((1, sh.bands_elems)), dtype=torch.float32, device="cuda")
+    nlev = sum(v ** 3 for v in sh.sides[:3])
+    got = {}
+    for g in (8, group):
+        plan = mods[1].Plan3D(sh, 1, group=g)
+        As, Aty = plan.analysis(s), plan.analysis_adjoint(y)
+        lhs = float(torch.dot(As[0].double(), y[0].double()))
+        rhs = float(torch.dot(s[0, :nlev].double(), Aty[0, :nlev].double()))
+        scale = float(As[0].double().norm() * y[0].double().norm())
+        assert abs(lhs - rhs) < TOL * scale, (g, lhs, rhs)
+        got[g] = Aty[0, :nlev].double()
+        plan.close()
+    assert float((got[group] - got[8]).abs().max() / got[8].abs().max()) < TOL
+    sh.close()
