@@ -3,9 +3,10 @@
 // The noise scalars of the denoise (shearlet_toolbox_1/nsst_scalars.m:28-45,
 // demo_denoise/shearcuda/shearcuda.cpp:205-271) are MAD/0.6745 of each band of
 // the transform of unit white noise.  The reference copies every band to the
-// host and takes two medians there; here one workgroup per plane finds the
-// order statistics by radix selection over monotone integer keys of the
-// values, so the result is the exact median of the data, as a sort gives it.
+// host and takes two medians there; here the order statistics are found by radix
+// selection over monotone integer keys of the values (one workgroup per plane, or
+// histograms split over many where a workspace is given and planes are large), so
+// the result is the exact median of the data, as a sort gives it.
 //
 // Two arithmetic conventions, each reproducing one caller bit for bit:
 //   SHX_MAD_FP64  values widened to double: m = (a + b) / 2 of the two middle

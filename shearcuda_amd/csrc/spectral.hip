@@ -1030,7 +1030,9 @@ __device__ __forceinline__ void col_block_order(int& tile, int& plane, int& img,
 // tiles back to back, so the scale spectrum tile (read by all bands of its
 // scale), each filter tile (read by the bands sharing it and by every image
 // of a batch) come from its L2 after the first read, and each line is fetched
-// once for the TG tiles that share it.  Measured against the tile-fastest
+// once for the TG tiles that share it (row-major spectra only; in strips of four
+// columns a tile's lines are its own, and the figures here are from before the
+// strips).  Measured against the tile-fastest
 // order of the other column passes: 512^2, 8 columns, 28.8 -> 24.8 us
 // (counted fetch 66 -> 47 MB); 1024^2, 8 columns, 91 -> 86 us; with the image
 // after the tile group instead of before the plane, the batched mix ran 1.5%
@@ -1183,9 +1185,10 @@ __global__ void __launch_bounds__(CT_ * Split<L>::R2) k_cols_rec(const float2* _
 }
 
 // ---------------------------------------------------------------------------
-// Column passes on the three-pass 512-point engine (fft3.h): eight values per
-// thread instead of sixteen, so the blocks hold far fewer registers and the
-// reconstruction keeps its running sum in registers (no second LDS tile).
+// Column passes on the engines with 64 threads per column (fft3.h, ColEng): half
+// the values per thread of the two-pass split (8 at 512, 16 at 1024), so the
+// blocks hold far fewer registers and the reconstruction keeps its running sum in
+// registers (no second LDS tile; 8 x 1024^2 denoise 2288 -> 2228 us).
 // Same grids, band maps and results (to FP32 rounding) as k_cols_dec<PRE> and
 // k_cols_rec.  Thread (c, tau) of a block of CT * 64 threads owns rows
 // tau + 64 s of tile column c.
@@ -2699,8 +2702,8 @@ hipError_t launch_dct_rec(int L, int step, const float2* Qg, long long qs, const
 }
 
 bool col_tile_ok(int L, int ct) {
-  // three-pass engines: 512 (8 x 8 x 8) with 4 or 8 columns, 1024
-  // (16 x 8 x 8 on 128 threads per column) with 2 or 4
+  // three-pass engines, 64 threads per column: 512 (8 x 8 x 8) with 4 or 8
+  // columns, 1024 (16 x 8 x 8) with 2 or 4
   if (ct < 0) return (L == 512 && (ct == -4 || ct == -8)) || (L == 1024 && (ct == -2 || ct == -4));
   switch (L) {
 #define SHX_CT_OK(LL) \
