@@ -491,6 +491,7 @@ int shx3_plan_create(const shx3_dict* d, int nvol, int group, shx3_plan** out) {
     const Level3& v = d->lv[l];
     const long long H = v.N / 2 + 1;
     sA = std::max(sA, group * H * v.n * v.n);
+    sA = std::max(sA, H * v.N * v.n);  // rows of inv3 from the padded grid (the transpose's sum)
     sB = std::max(sB, group * H * v.N * v.n);
     sS = std::max(sS, spec_elems(v.N));
   }

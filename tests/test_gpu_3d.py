@@ -323,3 +323,35 @@ def test_analysis_adjoint_at_ragged_groups(mods, n, dirs, mode, group):
         plan.close()
     assert float((got[group] - got[8]).abs().max() / got[8].abs().max()) < TOL
     sh.close()
+
+
+@pytest.mark.parametrize("n,dirs,mode", [(32, (2, 2, 2), 1), (48, (2, 2, 2), 1.5), (64, (2, 2, 2), 2)])
+def test_analysis_adjoint_one_band_per_group(mods, n, dirs, mode):
+    """Plans of one band per launch: the transpose's inverse runs from the
+    padded grid N > n, whose rows (H N n values a volume) are more than one
+    band's n^2 columns.  The workspace holds them, and a batch's volumes keep
+    apart: each equals the same volume through a plan of its own, bit for bit,
+    and the group of 8 to the rounding of a reordered FP32 sum."""
+    print("case adjoint group=1 n=%d" % n, flush=True)
+    sh = mods[1].Shear3D(n, dirs, mode)
+    nvol = 3
+    need = max((N // 2 + 1) * N * s for s, N in zip(sh.sides, sh.fft_sides))
+    spec = lambda N: (N // 2 + 1) * N * N
+    tB = max(spec(n), need)
+    rest = 4 * spec(n) + max(spec(N) for N in sh.fft_sides) + tB
+    plan = mods[1].Plan3D(sh, nvol, group=1)
+    assert plan.nbytes() >= nvol * (8 * (rest + need) + 2 * 4 * sh.subs_elems)
+    y = torch.tensor(np.random.default_rng(n).standard_normal((nvol, sh.bands_elems)), dtype=torch.float32,
+                     device="cuda")
+    nlev = sum(v ** 3 for v in sh.sides[:3])
+    got = plan.analysis_adjoint(y)[:, :nlev]
+    plan.close()
+    one = mods[1].Plan3D(sh, 1, group=1)
+    for i in range(nvol):
+        assert torch.equal(one.analysis_adjoint(y[i:i + 1].contiguous())[0, :nlev], got[i])
+    one.close()
+    wide = mods[1].Plan3D(sh, nvol, group=8)
+    ref = wide.analysis_adjoint(y)[:, :nlev].double()
+    assert float((got.double() - ref).abs().max() / ref.abs().max()) < TOL
+    wide.close()
+    sh.close()
