@@ -577,18 +577,19 @@ void stages_scale_fft(shx_dict* d, const Work& w, int nimg, hipStream_t s, std::
                 [=] { return shx::launch_cols_fwd(L, w.spec, w.s_spec / 2, S, nimg, d->tw, s, w.ct_dec); }});
 }
 
-void stage_cols_dec(shx_dict* d, const Work& w, int nimg, hipStream_t s, std::vector<Stage>& st) {
+// rows: the plain inverse row pass follows (a transform), not a fused one.
+void stage_cols_dec(shx_dict* d, const Work& w, int nimg, hipStream_t s, std::vector<Stage>& st, bool rows) {
   const int L = d->L, S = d->S, nb = d->nbands;
   const double P = 4.0 * L * L * nimg;
   st.push_back({"cols_dec", (S + 2.0 * nb) * P, [=] {
                   return shx::launch_cols_dec(L, w.spec, w.s_spec / 2, w.band, w.s_band / 2, d->Hmain, d->Hbeta,
-                                              w.map, nimg, d->tw, s, w.ct_dec, true);
+                                              w.map, nimg, d->tw, s, w.ct_dec, true, rows);
                 }});
 }
 
-void stages_spec_dec(shx_dict* d, const Work& w, int nimg, hipStream_t s, std::vector<Stage>& st) {
+void stages_spec_dec(shx_dict* d, const Work& w, int nimg, hipStream_t s, std::vector<Stage>& st, bool rows) {
   stages_scale_fft(d, w, nimg, s, st);
-  stage_cols_dec(d, w, nimg, s, st);
+  stage_cols_dec(d, w, nimg, s, st, rows);
 }
 
 // DCT-domain front end: the lowpass (c.low) and the scale spectra (w.spec)
@@ -620,14 +621,14 @@ void stages_dct_front(shx_dict* d, const Work& w, int nimg, const float* x, long
 // Decomposition up to the band spectra T (w.band): either front end, then the
 // column filter pass.
 void stages_front_dec(shx_dict* d, const Work& w, int nimg, const float* x, long long xs, const Coeffs& c,
-                      hipStream_t s, std::vector<Stage>& st) {
+                      hipStream_t s, std::vector<Stage>& st, bool rows) {
   if (w.dct_front) {
     stages_dct_front(d, w, nimg, x, xs, c, s, st);
   } else {
     stages_pyr_dec(d, w, nimg, x, xs, c, s, st);
     stages_scale_fft(d, w, nimg, s, st);
   }
-  stage_cols_dec(d, w, nimg, s, st);
+  stage_cols_dec(d, w, nimg, s, st, rows);
 }
 
 shx::ThreshSpec band_thresh(const shx_dict* d, const Thr& t) {
@@ -741,7 +742,7 @@ void stages_back_rec(shx_dict* d, const Work& w, int nimg, const Coeffs& c, cons
 // Forward transform: pyramid, spectral pass, band rows written to c.bands.
 void stages_dec(shx_dict* d, const Work& w, int nimg, const float* x, long long xs, const Coeffs& c, hipStream_t s,
                 std::vector<Stage>& st) {
-  stages_front_dec(d, w, nimg, x, xs, c, s, st);
+  stages_front_dec(d, w, nimg, x, xs, c, s, st, true);
   const int L = d->L, nb = d->nbands;
   const double P = 4.0 * L * L * nimg;
   PlaneSet bandset = shx::single_cell(reinterpret_cast<float*>(w.band), nb, w.s_band);
@@ -767,7 +768,7 @@ void stages_rec(shx_dict* d, const Work& w, int nimg, const Coeffs& c, const Thr
 // thresholded band row pass run as one kernel over each band row.
 void stages_denoise(shx_dict* d, const Work& w, int nimg, const float* x, long long xs, const Coeffs& c,
                     const Thr& t, float* out, long long os, hipStream_t s, std::vector<Stage>& st) {
-  stages_front_dec(d, w, nimg, x, xs, c, s, st);
+  stages_front_dec(d, w, nimg, x, xs, c, s, st, false);
   const int L = d->L, nb = d->nbands;
   const double P = 4.0 * L * L * nimg;
   PlaneSet bandset = shx::single_cell(reinterpret_cast<float*>(w.band), nb, w.s_band);
@@ -984,13 +985,13 @@ void stages_dec_adjoint_tail(shx_dict* d, const Work& w, int nimg, const Coeffs&
 
 // The pyramid part of S^T, up to the band spectra T (w.band).
 void stages_rec_adjoint_front(shx_dict* d, const Work& w, int nimg, const float* gx, long long gxs, const Coeffs& c,
-                              hipStream_t s, std::vector<Stage>& st) {
+                              hipStream_t s, std::vector<Stage>& st, bool rows) {
   if (w.dct_back && d->rmask) {
     stages_dct_front(d, w, nimg, gx, gxs, c, s, st, d->rmask);
-    stage_cols_dec(d, w, nimg, s, st);
+    stage_cols_dec(d, w, nimg, s, st, rows);
   } else {
     stages_pyr_rec_adjoint(d, w, nimg, gx, gxs, c, s, st);
-    stages_spec_dec(d, w, nimg, s, st);
+    stages_spec_dec(d, w, nimg, s, st, rows);
   }
 }
 
@@ -1011,7 +1012,7 @@ void stages_dec_adjoint(shx_dict* d, const Work& w, int nimg, const Coeffs& c, f
 // S^T: image gradient -> coefficient gradients.
 void stages_rec_adjoint(shx_dict* d, const Work& w, int nimg, const float* gx, long long gxs, const Coeffs& c,
                         hipStream_t s, std::vector<Stage>& st) {
-  stages_rec_adjoint_front(d, w, nimg, gx, gxs, c, s, st);
+  stages_rec_adjoint_front(d, w, nimg, gx, gxs, c, s, st, true);
   const int L = d->L, nb = d->nbands;
   const double P = 4.0 * L * L * nimg;
   PlaneSet bandset = shx::single_cell(reinterpret_cast<float*>(w.band), nb, w.s_band);
@@ -1034,7 +1035,7 @@ void stages_shrink_backward(shx_dict* d, const Work& w, int nimg, const Coeffs& 
   Coeffs g{};
   g.low = w.planes + (size_t)(S + 2) * pl;
   g.low_stride = w.s_planes;
-  stages_rec_adjoint_front(d, w, nimg, gout, gos, g, s, st);
+  stages_rec_adjoint_front(d, w, nimg, gout, gos, g, s, st, false);
   PlaneSet bandset = shx::single_cell(reinterpret_cast<float*>(w.band), nb, w.s_band);
   PlaneSet cb = c.bands;
   shx::ThreshSpec th = band_thresh(d, t);
@@ -1261,7 +1262,7 @@ int autotune_work(shx_dict* d, Work& w, int nimg, int reps, hipStream_t caller, 
     for (int c = 0; c < nct; ++c) {
       w.ct_dec = ccand[c];
       std::vector<Stage> st;
-      stages_spec_dec(d, w, nimg, s, st);
+      stages_spec_dec(d, w, nimg, s, st, false);
       const double t = time_stages_graph(st, s, reps);
       if (t > 0 && t < td[c]) td[c] = t;
     }
@@ -2355,7 +2356,7 @@ int shx_convolution(shx_dict* d, const float* const* y, float* const* coeff, voi
     SHX_HIP(hipMemcpyAsync(w.planes + (size_t)j * d->plane(), y[j + 1], pl, hipMemcpyDeviceToDevice, s));
   if (coeff[0] != y[0]) SHX_HIP(hipMemcpyAsync(coeff[0], y[0], pl, hipMemcpyDeviceToDevice, s));
   std::vector<Stage> st;
-  stages_spec_dec(d, w, 1, s, st);
+  stages_spec_dec(d, w, 1, s, st, true);
   const int L = d->L, nb = d->nbands;
   PlaneSet bandset = shx::single_cell(reinterpret_cast<float*>(w.band), nb, w.s_band);
   PlaneSet out = cell_coeffs(d, coeff).bands;

@@ -96,10 +96,11 @@ hipError_t launch_rows_c2r_mask_r2c(int L, const PlaneSet& Tin, const PlaneSet& 
                                     int nimg, const ThreshSpec& th, float* gth, const float2* tw, hipStream_t s);
 // ct: column tile width of the block (4, 8 or 16 where col_tile_ok; 0 = the
 // default for L).  pre: Y1 is already column-transformed (launch_cols_fwd).
+// rows: the plain inverse row pass (launch_rows_c2r) reads Tout next.
 bool col_tile_ok(int L, int ct);
 hipError_t launch_cols_dec(int L, const float2* Y1, long long y1_stride, float2* Tout, long long t_stride,
                            const float2* Hm, const float2* Hb, const BandMap& map, int nimg, const float2* tw,
-                           hipStream_t s, int ct = 0, bool pre = false);
+                           hipStream_t s, int ct = 0, bool pre = false, bool rows = false);
 // In-place forward column FFT of nplanes packed spectra (stride y1_stride per image).
 hipError_t launch_cols_fwd(int L, float2* Y1, long long y1_stride, int nplanes, int nimg, const float2* tw,
                            hipStream_t s, int ct = 0);

@@ -120,12 +120,10 @@ __device__ __forceinline__ float2 shfl2(float2 v, int src) {
   return make_float2(__shfl(v.x, src), __shfl(v.y, src));
 }
 
-// Band spectra are accessed non-temporally where one image's exceed the L2s (from
-// 512^2 on: 50 MB).  At 256^2 (12.6 MB) only the column passes' stores are, and
-// only in batches (48 x 256^2: 922 -> 875 us of kernels; one image, whose next
-// kernel reads them from the L2s: 84 us for the transform pair, non-temporal 86);
-// choosing the loads there at run time too broke up their batches (870 us a step
-// against 800).
+// Band spectra are accessed non-temporally from 512^2 on (50 MB for one image, more
+// than the L2s hold).  At 256^2 (12.6 MB) only the column passes' stores are, by the
+// bytes of the launch (band_nt below); choosing the loads there at run time too broke
+// up their batches (870 us a step of 48 images against 800).
 template <int L>
 __device__ __forceinline__ float2 band_ld(const float2* p) {
   return L >= 512 ? load_nt(p) : *p;
@@ -872,7 +870,7 @@ __device__ __forceinline__ void col_inv_B_to(const float2* buf, STORE store) {
 // Inverse column transform from pass-B layout registers (thread (c, k2)
 // holding Q[k2 + R2 k1]) to global.  Starts with a barrier
 // so buf may still be in use by the caller.  t: the first pass's twiddles
-// (col_inv_tw), loaded by the caller ahead of time.
+// (col_inv_tw), loaded by the caller ahead of time.  NT: non-temporal stores.
 template <int L>
 __device__ __forceinline__ PassTw<Split<L>::R1> col_inv_tw(int k2, const float2* __restrict__ tw) {
   PassTw<Split<L>::R1> t;
@@ -880,7 +878,7 @@ __device__ __forceinline__ PassTw<Split<L>::R1> col_inv_tw(int k2, const float2*
   return t;
 }
 
-template <int L, int CT_>
+template <int L, int CT_, bool NT>
 __device__ __forceinline__ void col_inv_from_B(float2 (&q)[Split<L>::R1], float2* __restrict__ dst, float2* buf,
                                                const PassTw<Split<L>::R1>& t) {
   using C = ColCfg<L, CT_>;
@@ -908,7 +906,7 @@ __device__ __forceinline__ void col_inv_from_B(float2 (&q)[Split<L>::R1], float2
     const unsigned lane = col_off<L>(kb + R1 * R1 * h, cp);
 #pragma unroll
     for (int k = 0; k < R1; ++k) {
-      if constexpr (L >= 512)
+      if constexpr (NT)
         bv.st2nt(w[k], lane, col_off<L>(R1 * k, 0));
       else
         bv.st2(w[k], lane, col_off<L>(R1 * k, 0));
@@ -924,12 +922,12 @@ __device__ __forceinline__ void col_inv_from_B(float2 (&q)[Split<L>::R1], float2
     dft<R2, +1>(w);
     const BufView bv = col_view<L, CT>(dst);
     const unsigned lane = col_off<L>(kb, c);
-    if (L >= 512 || (L == 256 && gridDim.z > 1)) {
 #pragma unroll
-      for (int k1 = 0; k1 < R2; ++k1) bv.st2nt(w[k1], lane, col_off<L>(R1 * k1, 0));
-    } else {
-#pragma unroll
-      for (int k1 = 0; k1 < R2; ++k1) bv.st2(w[k1], lane, col_off<L>(R1 * k1, 0));
+    for (int k1 = 0; k1 < R2; ++k1) {
+      if constexpr (NT)
+        bv.st2nt(w[k1], lane, col_off<L>(R1 * k1, 0));
+      else
+        bv.st2(w[k1], lane, col_off<L>(R1 * k1, 0));
     }
   }
 }
@@ -1079,7 +1077,7 @@ __global__ void __launch_bounds__(CT_ * Split<L>::R2) k_cols_fwd(float2* __restr
 
 // Column pass of the decomposition: one block per (column tile, band, image).
 // PRE: the scale spectrum is already column-transformed (k_cols_fwd).
-template <int L, int CT_, bool PRE>
+template <int L, int CT_, bool PRE, bool NT>
 __global__ void __launch_bounds__(CT_ * Split<L>::R2) k_cols_dec(const float2* __restrict__ Y1, long long y1_stride,
                                                             float2* __restrict__ Tout, long long t_stride,
                                                             const float2* __restrict__ Hmain,
@@ -1110,7 +1108,7 @@ __global__ void __launch_bounds__(CT_ * Split<L>::R2) k_cols_dec(const float2* _
     col_fwd_to_B<L, CT_>(u, src, buf, tw);
   }
   col_filter<L, CT_, false, false>(u, q, c0, h, Hbeta + (size_t)f * L, buf);
-  col_inv_from_B<L, CT_>(q, Tout + (size_t)b * t_stride + (size_t)p * L * NH + sp_ix<L>(0, c0), buf, ivt);
+  col_inv_from_B<L, CT_, NT>(q, Tout + (size_t)b * t_stride + (size_t)p * L * NH + sp_ix<L>(0, c0), buf, ivt);
 }
 
 // Column pass of the reconstruction: one block per (column tile, direction
@@ -1124,7 +1122,7 @@ struct ColRecAcc {
   static constexpr int SIZE = LDS ? ColCfg<L, CT_>::LDS : 1;
 };
 
-template <int L, int CT_>
+template <int L, int CT_, bool NT>
 __global__ void __launch_bounds__(CT_ * Split<L>::R2) k_cols_rec(const float2* __restrict__ U, long long u_stride,
                                                             float2* __restrict__ Q, long long q_stride,
                                                             const float2* __restrict__ Hmain,
@@ -1181,7 +1179,8 @@ __global__ void __launch_bounds__(CT_ * Split<L>::R2) k_cols_rec(const float2* _
 #pragma unroll
     for (int k1 = 0; k1 < R1; ++k1) acc[k1] = row[k1 * (R2 / R1) * C::Lds::BLK];
   }
-  col_inv_from_B<L, CT_>(acc, Q + (size_t)b * q_stride + (size_t)g * L * NH + sp_ix<L>(0, c0), buf, col_inv_tw<L>(k2, tw));
+  col_inv_from_B<L, CT_, NT>(acc, Q + (size_t)b * q_stride + (size_t)g * L * NH + sp_ix<L>(0, c0), buf,
+                             col_inv_tw<L>(k2, tw));
 }
 
 // ---------------------------------------------------------------------------
@@ -1192,7 +1191,7 @@ __global__ void __launch_bounds__(CT_ * Split<L>::R2) k_cols_rec(const float2* _
 // Same grids, band maps and results (to FP32 rounding) as k_cols_dec<PRE> and
 // k_cols_rec.  Thread (c, tau) of a block of CT * 64 threads owns rows
 // tau + 64 s of tile column c.
-template <int L, int CT>
+template <int L, int CT, bool NT>
 __global__ void __launch_bounds__(CT * 64) k_cols_dec3(const float2* __restrict__ Y1, long long y1_stride,
                                                    float2* __restrict__ Tout, long long t_stride,
                                                    const float2* __restrict__ Hmain, const float2* __restrict__ Hbeta,
@@ -1235,7 +1234,12 @@ __global__ void __launch_bounds__(CT * 64) k_cols_dec3(const float2* __restrict_
   G::template fft<+1>(q, buf, t);
   const BufView tv = col_view<L, CT>(Tout + (size_t)b * t_stride + (size_t)p * L * NH + sp_ix<L>(0, c0));
 #pragma unroll
-  for (int k = 0; k < NV; ++k) tv.st2nt(q[k], lane, col_off<L>(64 * k, 0));
+  for (int k = 0; k < NV; ++k) {
+    if constexpr (NT)
+      tv.st2nt(q[k], lane, col_off<L>(64 * k, 0));
+    else
+      tv.st2(q[k], lane, col_off<L>(64 * k, 0));
+  }
 }
 
 template <int L, int CT>
@@ -1360,16 +1364,45 @@ struct Launch {
                        tw);
     return hipGetLastError();
   }
+  // Whether a column pass stores its spectra non-temporally (graph replays, us).
+  // 256^2: from 480 planes (120 MB) in one launch on.  Below that what follows reads
+  // them faster from the caches (8 images, denoise with coefficients 183 non-temporal,
+  // 175 not; 4 images, transform 62.3 and 60.8; a plan of one launch per scale, whose
+  // launches are a third as large: 16 images 434 and 406); above it they push out what
+  // the blocks share (16 images in one launch 341 and 359, 20 images 426 and 435).
+  // 512^2: always, but for one image whose planes go straight to the plain row pass
+  // (rows: transform 80 non-temporal, 76.5 not; image-only denoise 113.5 and 114.4).
+  // 1024^2: always (4 images, denoise 1131 against 1425 with every access cached and
+  // rows not in strips).
+  static bool band_nt(const BandMap& map, int nimg, bool rows) {
+    if (L == 512) return !(rows && nimg == 1);
+    return L >= 1024 || (L == 256 && map.nbands * (long long)nimg >= 480);
+  }
+  // Calls fn with band_nt's answer as a type; a size has the forms its rule can choose.
+  template <class F>
+  static void by_nt(bool nt, F fn) {
+    if constexpr (L >= 1024) {
+      fn(std::true_type{});
+    } else if constexpr (L < 256) {
+      fn(std::false_type{});
+    } else {
+      if (nt)
+        fn(std::true_type{});
+      else
+        fn(std::false_type{});
+    }
+  }
   template <int CT>
   static hipError_t cols_dec_ct(const float2* Y1, long long ys, float2* To, long long ts, const float2* Hm,
                                 const float2* Hb, const BandMap& map, int nimg, const float2* tw, hipStream_t s,
-                                bool pre) {
-    if (pre)
-      hipLaunchKernelGGL((k_cols_dec<L, CT, true>), dim3(L / 2 / CT, map.nbands, nimg), dim3(ColCfg<L, CT>::T), 0, s,
-                         Y1, ys, To, ts, Hm, Hb, map, tw);
-    else
-      hipLaunchKernelGGL((k_cols_dec<L, CT, false>), dim3(L / 2 / CT, map.nbands, nimg), dim3(ColCfg<L, CT>::T), 0,
-                         s, Y1, ys, To, ts, Hm, Hb, map, tw);
+                                bool pre, bool rows) {
+    const dim3 grid(L / 2 / CT, map.nbands, nimg), blk(ColCfg<L, CT>::T);
+    by_nt(band_nt(map, nimg, rows), [&](auto nt) {
+      if (pre)
+        hipLaunchKernelGGL((k_cols_dec<L, CT, true, nt.value>), grid, blk, 0, s, Y1, ys, To, ts, Hm, Hb, map, tw);
+      else
+        hipLaunchKernelGGL((k_cols_dec<L, CT, false, nt.value>), grid, blk, 0, s, Y1, ys, To, ts, Hm, Hb, map, tw);
+    });
     return hipGetLastError();
   }
   template <int CT>
@@ -1381,16 +1414,21 @@ struct Launch {
   template <int CT>
   static hipError_t cols_rec_ct(const float2* U, long long us, float2* Q, long long qs, const float2* Hm,
                                 const float2* Hb, const BandMap& map, int nimg, const float2* tw, hipStream_t s) {
-    hipLaunchKernelGGL((k_cols_rec<L, CT>), dim3(L / 2 / CT, map.ngroups, nimg), dim3(ColCfg<L, CT>::T), 0, s, U, us,
-                       Q, qs, Hm, Hb, map, tw);
+    const dim3 grid(L / 2 / CT, map.ngroups, nimg), blk(ColCfg<L, CT>::T);
+    by_nt(band_nt(map, nimg, false), [&](auto nt) {
+      hipLaunchKernelGGL((k_cols_rec<L, CT, nt.value>), grid, blk, 0, s, U, us, Q, qs, Hm, Hb, map, tw);
+    });
     return hipGetLastError();
   }
   template <int CT>
   static hipError_t cols_dec3_ct(const float2* Y1, long long ys, float2* To, long long ts, const float2* Hm,
-                                 const float2* Hb, const BandMap& map, int nimg, const float2* tw, hipStream_t s) {
+                                 const float2* Hb, const BandMap& map, int nimg, const float2* tw, hipStream_t s,
+                                 bool rows) {
     if constexpr ((L == 512 && CT >= 4) || L == 1024)
-      hipLaunchKernelGGL((k_cols_dec3<L, CT>), dim3(L / 2 / CT, map.nbands, nimg), dim3(CT * 64), 0, s, Y1, ys, To,
-                         ts, Hm, Hb, map, tw);
+      by_nt(band_nt(map, nimg, rows), [&](auto nt) {
+        hipLaunchKernelGGL((k_cols_dec3<L, CT, nt.value>), dim3(L / 2 / CT, map.nbands, nimg), dim3(CT * 64), 0, s, Y1,
+                           ys, To, ts, Hm, Hb, map, tw);
+      });
     return hipGetLastError();
   }
   template <int CT>
@@ -1414,20 +1452,20 @@ struct Launch {
   static constexpr int kDefaultTile = ColTile<L>::narrow ? 4 : (ColTile<L>::dflt < 8 ? ColTile<L>::dflt : 8);
   static hipError_t cols_dec(const float2* Y1, long long ys, float2* To, long long ts, const float2* Hm,
                              const float2* Hb, const BandMap& map, int nimg, const float2* tw, hipStream_t s, int ct,
-                             bool pre) {
+                             bool pre, bool rows) {
     if (ct < 0) {
       if ((L != 512 && L != 1024) || !pre) return hipErrorInvalidValue;
-      if (ct == -2 && L == 1024) return cols_dec3_ct<2>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s);
-      if (ct == -4) return cols_dec3_ct<4>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s);
-      if (ct == -8) return cols_dec3_ct<8>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s);
+      if (ct == -2 && L == 1024) return cols_dec3_ct<2>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, rows);
+      if (ct == -4) return cols_dec3_ct<4>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, rows);
+      if (ct == -8) return cols_dec3_ct<8>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, rows);
       return hipErrorInvalidValue;
     }
     if (ct == 0) ct = kDefaultTile;
     if (ct == 4 && ColTile<L>::narrow)
-      return cols_dec_ct<(ColTile<L>::narrow ? 4 : 8)>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, pre);
-    if (ct == 8) return cols_dec_ct<8>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, pre);
+      return cols_dec_ct<(ColTile<L>::narrow ? 4 : 8)>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, pre, rows);
+    if (ct == 8) return cols_dec_ct<8>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, pre, rows);
     if (ct == 16 && ColTile<L>::wide)
-      return cols_dec_ct<(ColTile<L>::wide ? 16 : 8)>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, pre);
+      return cols_dec_ct<(ColTile<L>::wide ? 16 : 8)>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, pre, rows);
     return hipErrorInvalidValue;
   }
   static hipError_t cols_fwd(float2* Y1, long long ys, int nplanes, int nimg, const float2* tw, hipStream_t s, int ct) {
@@ -1489,8 +1527,8 @@ hipError_t launch_rows_c2r_mask_r2c(int L, const PlaneSet& Tin, const PlaneSet& 
 
 hipError_t launch_cols_dec(int L, const float2* Y1, long long ys, float2* To, long long ts, const float2* Hm,
                            const float2* Hb, const BandMap& map, int nimg, const float2* tw, hipStream_t s, int ct,
-                           bool pre) {
-  SHX_BY_L(L, LT::cols_dec(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, ct, pre))
+                           bool pre, bool rows) {
+  SHX_BY_L(L, LT::cols_dec(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, ct, pre, rows))
 }
 
 hipError_t launch_cols_fwd(int L, float2* Y1, long long ys, int nplanes, int nimg, const float2* tw, hipStream_t s,

@@ -256,6 +256,33 @@ def test_batch_matches_plain(api, L, nimg):
     shear.close()
 
 
+@pytest.mark.parametrize("L,nimg,part,ct", [(256, 10, 5, 0), (256, 10, 5, 8), (512, 2, 1, 0), (512, 2, 1, 8), (512, 2, 1, -4)])
+def test_batch_equals_its_parts_across_the_store_rule(api, L, nimg, part, ct):
+    """Band spectra leave the decomposition's column pass non-temporally from
+    480 planes of 256^2 in a launch on, and at 512^2 but for one image's
+    transform: the same images on both sides of the rule give the same bits."""
+    print("case store rule L=%d nimg=%d ct=%d" % (L, nimg, ct), flush=True)
+    shear = api.make_dictionary(L)
+    xg = to_gpu(np.stack([image(L, seed=90 + i)[1] for i in range(nimg)]))
+    th = torch.full((nimg, shear.nbands), 40.0, device="cuda")
+
+    def run(x, t):
+        b = api.Batch(shear, x.shape[0])
+        api.set_schedule(shear, 0, 4, batch=b, col_tile_dec=ct)
+        api.set_plan_options(shear, b, dct_front=True, dct_back=True)
+        c1, c2, out = b.alloc_coeffs(), b.alloc_coeffs(), torch.empty_like(x)
+        b.shear_trans(x, c1)
+        b.denoise(x, c2, t, out)
+        torch.cuda.synchronize()
+        b.close()
+        return c1, c2, out
+    whole = run(xg, th)
+    for i in range(0, nimg, part):
+        for got, ref in zip(run(xg[i:i + part].contiguous(), th[i:i + part].contiguous()), whole):
+            assert torch.equal(got, ref[i:i + part])
+    shear.close()
+
+
 @pytest.mark.parametrize("parallel", [False, True])
 def test_mixed_size_batches_in_one_graph(api, parallel):
     print("case mixed graph parallel=%s" % parallel, flush=True)
