@@ -274,13 +274,17 @@ __global__ void __launch_bounds__(MT) k_band_mad(const float* __restrict__ plane
 //   k_mad_hist    histogram of the keys' top 12 bits, per block
 //   k_mad_find    one block per plane: the bin of the middle rank
 //   k_mad_hist    the next 11 bits inside that bin; returns at once for a plane
-//                 whose bin already fits the candidate buffer (every band of a
-//                 transform does: a bin is an eighth of an octave)
+//                 whose bin already fits the candidate buffer.  A bin is an eighth
+//                 of an octave and holds 3 to 5% of a Gaussian plane at the median
+//                 of its deviations: planes of up to 512^2 fit, 1024^2 planes and
+//                 128^3 bands mostly do not.
+//   k_mad_find    the bin among those 11 bits (where find2_in_gather is false; else
+//                 every block of the gather finds it itself)
 //   k_mad_gather  values of the bin to the candidate buffer, and the smallest
 //                 key above the bin
 //   k_mad_select  one block per plane: exact selection among the candidates,
 //                 in LDS
-// so the plane is read twice per median, by all CUs: 92 us for the same
+// so the plane is read two or three times per median, by all CUs: 92 us for the same
 // planes, bound by the latency of ten short dependent launches (the four
 // streaming ones read 51 MB in 11-15 us each).  The 64-bit deviations
 // are binned by their float rounding, which keeps their order, and compared
@@ -294,10 +298,10 @@ constexpr int SCHUNK = 16384, GCHUNK = 8192;         // elements per block
 static_assert(HBINS == 4 * MT && H2BINS == 2 * MT && ST == MT / 2, "bin scans of the streaming kernels");
 
 struct MadState {
-  uint32_t prefix, rank;    // first bin of the middle rank, and the rank inside it
-  uint32_t rank2;           // the rank inside the final bin
+  uint32_t prefix, shift;   // bin of the middle rank: the keys with key >> shift == prefix
+  uint32_t rank;            // the rank inside the bin
+  uint32_t rank2;           // the rank inside the gathered bin
   uint32_t second, ncand;   // the second histogram was needed; candidates
-  uint32_t pad;
   double m;                 // out: the median of the values
 };
 
@@ -395,35 +399,53 @@ __global__ void __launch_bounds__(ST) k_mad_hist(MadPlanes io) {
   for (int i = threadIdx.x; i < NB / 2; i += ST) mine[i] = hist[2 * i] | (hist[2 * i + 1] << 16);
 }
 
-// The bin of the plane's middle rank, and the start values of the gather.
-template <int STAGE>
+// The bin of the plane's middle rank, and the start values of the gather; SECOND:
+// the bin inside that one.
+template <int STAGE, bool SECOND>
 __global__ void __launch_bounds__(ST) k_mad_find(MadPlanes io) {
   __shared__ uint32_t wsum[ST / 64], res[3];
-  const uint32_t rank = (uint32_t)((io.n - 1) / 2);
-  find_bin_parts<HBINS / ST>(io.part + (size_t)blockIdx.x * io.gh * HBINS, io.gh, rank, wsum, res);
-  if (threadIdx.x == 0) {
-    MadState* st = io.st + 2 * blockIdx.x + STAGE;
-    st->prefix = res[0];
-    st->rank = rank - res[1];
-    st->second = res[2] > (uint32_t)MCAP;
-    st->ncand = 0;
+  MadState* st = io.st + 2 * blockIdx.x + STAGE;
+  const uint16_t* part = io.part + (size_t)blockIdx.x * io.gh * HBINS;
+  if constexpr (SECOND) {
+    if (!st->second) return;
+    const uint32_t rank = st->rank;
+    find_bin_parts<H2BINS / ST>(part, io.gh, rank, wsum, res);
+    if (threadIdx.x == 0) {
+      st->prefix = (st->prefix << H2BITS) | res[0];
+      st->shift -= H2BITS;
+      st->rank = rank - res[1];
+    }
+  } else {
+    const uint32_t rank = (uint32_t)((io.n - 1) / 2);
+    find_bin_parts<HBINS / ST>(part, io.gh, rank, wsum, res);
+    if (threadIdx.x == 0) {
+      st->prefix = res[0];
+      st->shift = 32 - HBITS;
+      st->rank = rank - res[1];
+      st->second = res[2] > (uint32_t)MCAP;
+      st->ncand = 0;
+    }
   }
 }
 
-template <int STAGE, bool VEC, bool FP32>
+// FIND2: a block adds up the plane's second histograms itself instead of a launch of
+// k_mad_find before the gather.
+template <int STAGE, bool VEC, bool FP32, bool FIND2>
 __global__ void __launch_bounds__(ST) k_mad_gather(MadPlanes io) {
   __shared__ float buf[GCHUNK];
   __shared__ uint32_t cnt, base;
   __shared__ uint64_t mn[ST / 64];
-  __shared__ uint32_t wsum[ST / 64], res[3];
   MadState* st = io.st + 2 * blockIdx.y + STAGE;
   const MadKey<STAGE, FP32> kf{STAGE ? io.st[2 * blockIdx.y].m : 0.0};
-  uint32_t prefix = st->prefix, rank = st->rank, shift = 32 - HBITS;
-  if (st->second) {
-    find_bin_parts<H2BINS / ST>(io.part + (size_t)blockIdx.y * io.gh * HBINS, io.gh, rank, wsum, res);
-    prefix = (prefix << H2BITS) | res[0];
-    rank -= res[1];
-    shift -= H2BITS;
+  uint32_t prefix = st->prefix, rank = st->rank, shift = st->shift;
+  if constexpr (FIND2) {
+    __shared__ uint32_t wsum[ST / 64], res[3];
+    if (st->second) {
+      find_bin_parts<H2BINS / ST>(io.part + (size_t)blockIdx.y * io.gh * HBINS, io.gh, rank, wsum, res);
+      prefix = (prefix << H2BITS) | res[0];
+      rank -= res[1];
+      shift -= H2BITS;
+    }
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) st->rank2 = rank;
   if (threadIdx.x == 0) cnt = 0;
@@ -500,13 +522,29 @@ __global__ void __launch_bounds__(MT) k_mad_select(MadPlanes io, double* __restr
   }
 }
 
+// Whether the gather's blocks each add up the plane's second histograms (gh of 4 KB).
+// A launch of k_mad_find instead costs 2-3 us, also where no plane needs the second
+// histogram (up to 512^2: 49 planes 91 us); the sums of all blocks grow with the
+// square of a plane's size.  In the gather for planes of up to 512^2 and while all
+// sums are at most 64 MB (one 1024^2 plane 68 us, with the launch 72); beyond, the
+// launch: 49 x 1024^2 282 -> 220 us, 192 x 128^3 2964 -> 1670, 2^27 elements 31.6 ->
+// 3.9 ms.
+bool find2_in_gather(const MadPlanes& io, int nplanes) {
+  return io.gh <= 16 || (long long)io.gh * io.gg * nplanes <= 16384;
+}
+
 template <int STAGE, bool VEC, bool FP32>
 void launch_mad_stage(const MadPlanes& io, int nplanes, double* mad, hipStream_t s) {
   const dim3 gh(io.gh, nplanes), gg(io.gg, nplanes);
   hipLaunchKernelGGL((k_mad_hist<STAGE, VEC, FP32, false>), gh, dim3(ST), 0, s, io);
-  hipLaunchKernelGGL((k_mad_find<STAGE>), dim3(nplanes), dim3(ST), 0, s, io);
+  hipLaunchKernelGGL((k_mad_find<STAGE, false>), dim3(nplanes), dim3(ST), 0, s, io);
   hipLaunchKernelGGL((k_mad_hist<STAGE, VEC, FP32, true>), gh, dim3(ST), 0, s, io);
-  hipLaunchKernelGGL((k_mad_gather<STAGE, VEC, FP32>), gg, dim3(ST), 0, s, io);
+  if (find2_in_gather(io, nplanes)) {
+    hipLaunchKernelGGL((k_mad_gather<STAGE, VEC, FP32, true>), gg, dim3(ST), 0, s, io);
+  } else {
+    hipLaunchKernelGGL((k_mad_find<STAGE, true>), dim3(nplanes), dim3(ST), 0, s, io);
+    hipLaunchKernelGGL((k_mad_gather<STAGE, VEC, FP32, false>), gg, dim3(ST), 0, s, io);
+  }
   hipLaunchKernelGGL((k_mad_select<STAGE, VEC, FP32>), dim3(nplanes), dim3(MT), 0, s, io, mad);
 }
 

@@ -157,3 +157,43 @@ def test_band_mad_split_planes(gpu, n, kind):
         got = api.band_mad_cuda(t, arith).cpu().numpy()
         want = np.array([ref(r) for r in a])
         assert np.array_equal(got, want), (arith, got, want)
+
+
+def test_band_mad_time_is_linear_in_the_plane(gpu):
+    """One plane of normal values, whose middle bin needs the second histogram,
+    four times as large: about four times the time (every pass is linear),
+    where a sum over the plane's histograms in every block made it eleven."""
+    from shearcuda_amd import api
+    gen = torch.Generator("cuda").manual_seed(3)
+    ms = {}
+    for e in (24, 26):
+        x = torch.randn(1, 1 << e, device="cuda", generator=gen)
+        api.band_mad_cuda(x)
+        ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        best = float("inf")
+        for _ in range(10):
+            ev[0].record()
+            api.band_mad_cuda(x)
+            ev[1].record()
+            torch.cuda.synchronize()
+            best = min(best, ev[0].elapsed_time(ev[1]))
+        ms[e] = best
+    print("MAD of 2^24 and 2^26 elements: %.3f and %.3f ms" % (ms[24], ms[26]), flush=True)
+    assert ms[26] < 7 * ms[24]
+
+
+@pytest.mark.parametrize("nplanes,n", [(2, 262144), (2, 262145), (1, 1 << 20), (3, 1 << 20)])
+@pytest.mark.parametrize("kind", ["offset", "normal"])
+def test_band_mad_second_bin_forms(gpu, nplanes, n, kind):
+    """Both places that find the bin of the second histogram (a launch of its
+    own, every block of the gather), on both sides of their rule, with planes
+    that need it and planes that do not in one call."""
+    from shearcuda_amd import api
+    a = np.random.default_rng(n + nplanes).standard_normal((nplanes, n))
+    if kind == "offset":  # the first plane needs it for its values too
+        a[0] += 140.0
+    a = a.astype(np.float32)
+    t = torch.from_numpy(a).cuda()
+    for arith, ref in (("fp64", _mad64), ("fp32", _mad32)):
+        got = api.band_mad_cuda(t, arith).cpu().numpy()
+        assert np.array_equal(got, np.array([ref(r) for r in a])), arith
