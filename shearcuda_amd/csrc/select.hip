@@ -58,14 +58,15 @@ struct KeyDev32 {
   __device__ uint64_t operator()(float v) const { return __float_as_uint(fabsf(v - m)); }
 };
 
-// Calls fn(v) for every element of p[0, n) over the block's NT threads.
+// Calls fn(v) for every element of p[0, n) over the block's NT threads.  Unsigned
+// indices: the step past the end of a plane of 2^31 - 1 elements exceeds an int.
 template <bool VEC, int NT, class F>
-__device__ __forceinline__ void each_value(const float* __restrict__ p, int n, F&& fn) {
-  int i0 = 0;
+__device__ __forceinline__ void each_value(const float* __restrict__ p, uint32_t n, F&& fn) {
+  uint32_t i0 = 0;
   if constexpr (VEC) {
     const float4* p4 = reinterpret_cast<const float4*>(p);
-    const int n4 = n >> 2;
-    int i = threadIdx.x;
+    const uint32_t n4 = n >> 2;
+    uint32_t i = threadIdx.x;
     // four loads in flight: fn's LDS atomics keep the compiler from moving
     // the next load above them
     for (; i + 3 * NT < n4; i += 4 * NT) {
@@ -89,7 +90,7 @@ __device__ __forceinline__ void each_value(const float* __restrict__ p, int n, F
     }
     i0 = n4 << 2;
   }
-  for (int i = i0 + threadIdx.x; i < n; i += NT) fn(p[i]);
+  for (uint32_t i = i0 + threadIdx.x; i < n; i += NT) fn(p[i]);
 }
 
 struct SelShared {
@@ -304,6 +305,20 @@ struct MadState {
   uint32_t second, ncand;   // the second histogram was needed; candidates
   double m;                 // out: the median of the values
 };
+
+// Blocks of a plane's histogram and gather passes (planes of up to 2^31 - 1 elements,
+// so the rounding is done in 64 bits).
+struct MadBlocks {
+  int gh, gg;
+  constexpr explicit MadBlocks(long long n)
+      : gh((int)((n + SCHUNK - 1) / SCHUNK)), gg((int)((n + GCHUNK - 1) / GCHUNK)) {}
+  // workspace bytes of one plane
+  constexpr size_t bytes() const {
+    return 2 * sizeof(MadState) + sizeof(float) * MCAP + sizeof(uint16_t) * HBINS * (size_t)gh +
+           sizeof(uint64_t) * (size_t)gg;
+  }
+};
+static_assert(MadBlocks(0x7fffffff).gh == 131072 && MadBlocks(0x7fffffff).gg == 262144, "the largest plane");
 
 struct MadPlanes {
   const float* p;
@@ -560,7 +575,8 @@ void launch_mad(const float* planes, long long stride, int n, int nplanes, doubl
     return;
   }
   // grid.y holds at most 65535 planes
-  const int gh = (n + SCHUNK - 1) / SCHUNK, gg = (n + GCHUNK - 1) / GCHUNK;
+  const MadBlocks mb(n);
+  const int gh = mb.gh, gg = mb.gg;
   MadState* st = static_cast<MadState*>(work);
   float* cand = reinterpret_cast<float*>(st + 2 * (size_t)nplanes);
   uint16_t* part = reinterpret_cast<uint16_t*>(cand + (size_t)nplanes * MCAP);
@@ -579,9 +595,7 @@ void launch_mad(const float* planes, long long stride, int n, int nplanes, doubl
 extern "C" size_t shx_band_mad_workspace(long long plane_elems, int nplanes) {
   using namespace shx;
   if (plane_elems <= MCAP || nplanes < 1) return 0;
-  const size_t gh = (size_t)((plane_elems + SCHUNK - 1) / SCHUNK), gg = (size_t)((plane_elems + GCHUNK - 1) / GCHUNK);
-  return (size_t)nplanes * (2 * sizeof(MadState) + sizeof(float) * MCAP + sizeof(uint16_t) * HBINS * gh +
-                            sizeof(uint64_t) * gg);
+  return (size_t)nplanes * MadBlocks(plane_elems).bytes();
 }
 
 extern "C" int shx_band_mad_ws(const float* planes, long long plane_elems, long long plane_stride, int nplanes,

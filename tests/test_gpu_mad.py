@@ -197,3 +197,26 @@ def test_band_mad_second_bin_forms(gpu, nplanes, n, kind):
     for arith, ref in (("fp64", _mad64), ("fp32", _mad32)):
         got = api.band_mad_cuda(t, arith).cpu().numpy()
         assert np.array_equal(got, np.array([ref(r) for r in a])), arith
+
+
+def test_band_mad_of_the_largest_plane(gpu):
+    """2^31 - 1 elements, the largest plane the entry point takes: 24-bit whole
+    numbers in a scrambled order, each 128 times but one, so both medians are
+    known exactly.  Block counts, index steps past the end and workspace
+    offsets have to hold in their types; the many equal values send both
+    selections through the plane itself."""
+    from shearcuda_amd import api
+    n, a, chunk = (1 << 31) - 1, 1103515245, 1 << 27   # a odd: i -> a i mod 2^31 is a permutation
+    t = torch.empty(1, n, device="cuda")
+    for c in range(0, n, chunk):
+        i = torch.arange(c, min(n, c + chunk), device="cuda")
+        t[0, c:c + chunk] = ((i * a) & ((1 << 31) - 1)) >> 7
+    del i
+    count = np.full(1 << 24, 128, dtype=np.int64)
+    count[(((1 << 31) - 1) * a % (1 << 31)) >> 7] -= 1   # the index the plane stops short of
+    mid = (n - 1) // 2
+    m = int(np.searchsorted(np.cumsum(count), mid, side="right"))
+    dev = np.bincount(np.abs(np.arange(1 << 24) - m), weights=count).astype(np.int64)
+    want = int(np.searchsorted(np.cumsum(dev), mid, side="right")) / 0.6745
+    print("case largest plane", flush=True)
+    assert float(api.band_mad_cuda(t, "fp32")[0]) == want
