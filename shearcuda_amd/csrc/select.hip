@@ -58,27 +58,28 @@ struct KeyDev32 {
   __device__ uint64_t operator()(float v) const { return __float_as_uint(fabsf(v - m)); }
 };
 
-// Calls fn(v) for every element of p[0, n) over the block's NT threads.  Unsigned
-// indices: the step past the end of a plane of 2^31 - 1 elements exceeds an int.
-template <bool VEC, int NT, class F>
-__device__ __forceinline__ void each_value(const float* __restrict__ p, uint32_t n, F&& fn) {
-  uint32_t i0 = 0;
+// Calls fn(v) for every element of p[0, n) over the block's NT threads.
+// U: float4 loads in flight (fn's LDS atomics keep the compiler from moving the next
+// load above them); one for planes of a few thousand elements, which have no more
+// (16384 planes of 1024: 472 us, four 499; 49 planes of 1024^2, four 702 us, one 962).
+template <bool VEC, int NT, int U, class F>
+__device__ __forceinline__ void each_value(const float* __restrict__ p, int n, F&& fn) {
   if constexpr (VEC) {
     const float4* p4 = reinterpret_cast<const float4*>(p);
-    const uint32_t n4 = n >> 2;
-    uint32_t i = threadIdx.x;
-    // four loads in flight: fn's LDS atomics keep the compiler from moving
-    // the next load above them
-    for (; i + 3 * NT < n4; i += 4 * NT) {
-      float4 v[4];
+    const int n4 = n >> 2;
+    int i = threadIdx.x;
+    if constexpr (U > 1) {
+      for (; i + (U - 1) * NT < n4; i += U * NT) {
+        float4 v[U];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) v[u] = p4[i + u * NT];
+        for (int u = 0; u < U; ++u) v[u] = p4[i + u * NT];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        fn(v[u].x);
-        fn(v[u].y);
-        fn(v[u].z);
-        fn(v[u].w);
+        for (int u = 0; u < U; ++u) {
+          fn(v[u].x);
+          fn(v[u].y);
+          fn(v[u].z);
+          fn(v[u].w);
+        }
       }
     }
     for (; i < n4; i += NT) {
@@ -88,9 +89,12 @@ __device__ __forceinline__ void each_value(const float* __restrict__ p, uint32_t
       fn(v.z);
       fn(v.w);
     }
-    i0 = n4 << 2;
+    const int rest = n & 3;
+    if ((int)threadIdx.x < rest) fn(p[n - rest + threadIdx.x]);
+  } else {
+    // unsigned: the step past the end of a plane of 2^31 - 1 elements exceeds an int
+    for (uint32_t i = threadIdx.x; i < (uint32_t)n; i += NT) fn(p[i]);
   }
-  for (uint32_t i = i0 + threadIdx.x; i < n; i += NT) fn(p[i]);
 }
 
 struct SelShared {
@@ -149,16 +153,16 @@ __device__ __forceinline__ void block_minmax(uint64_t& mn, uint64_t& mx, SelShar
   __syncthreads();
 }
 
-// Key of the element of rank k (0-based) of p[0, n) under kf; *after_eq is
-// the number of elements with the same key ranked after it.  All keys lie in
-// [kmin, kmax], so the passes start at the highest bit in which these differ.
-template <bool VEC, class K>
-__device__ uint64_t block_select(const float* __restrict__ p, int n, uint32_t k, const K& kf, uint64_t kmin,
-                                 uint64_t kmax, SelShared& sh, uint32_t* after_eq) {
+// Key of the element of rank k (0-based) of p[0, n) under kf, all of whose keys agree
+// above their low `top` bits (there: `above`); *after_eq is the number of elements with
+// the same key ranked after it.  W: `top` at compile time (whole planes, whose passes
+// then unroll with constant masks: 4096 planes of 4096 331 -> 216 us), or 0.
+template <bool VEC, int U, int W, class K>
+__device__ uint64_t block_select(const float* __restrict__ p, int n, uint32_t k, const K& kf, int top, uint64_t above,
+                                 SelShared& sh, uint32_t* after_eq) {
   const int t = threadIdx.x;
-  const int top = kmin == kmax ? 0 : 64 - __clzll((long long)(kmin ^ kmax));
-  uint64_t pmask = top == 64 ? 0 : ~0ull << top;
-  uint64_t prefix = kmin & pmask;
+  if constexpr (W > 0) top = W, above = 0;
+  uint64_t prefix = above, pmask = W > 0 || top == 64 ? 0 : ~0ull << top;
   uint32_t krem = k, cnt = (uint32_t)n;
   for (int left = top; left > 0;) {
     const int d = left < MBITS ? left : MBITS;
@@ -167,7 +171,7 @@ __device__ uint64_t block_select(const float* __restrict__ p, int n, uint32_t k,
     sh.hist[2 * t] = 0;
     sh.hist[2 * t + 1] = 0;
     __syncthreads();
-    each_value<VEC, MT>(p, n, [&](float v) {
+    each_value<VEC, MT, U>(p, n, [&](float v) {
       const uint64_t key = kf(v);
       if ((key & pmask) == prefix) atomicAdd(&sh.hist[(uint32_t)(key >> shift) & dmask], 1u);
     });
@@ -184,35 +188,27 @@ __device__ uint64_t block_select(const float* __restrict__ p, int n, uint32_t k,
   return prefix;
 }
 
-// The keys of ranks k and k + 1 (the latter only if `two`) of p[0, n); `above`
-// is the smallest key past the array (the answer if rank k is its last).
-template <bool VEC, class K>
-__device__ void block_pair(const float* __restrict__ p, int n, uint32_t k, bool two, uint64_t above, const K& kf,
-                           uint64_t kmin, uint64_t kmax, SelShared& sh, uint64_t* lo, uint64_t* hi) {
-  uint32_t after = 0;
-  *lo = *hi = block_select<VEC>(p, n, k, kf, kmin, kmax, sh, &after);
-  if (!two || after > 0) return;
-  uint64_t mn = above, mx = 0;
-  each_value<VEC, MT>(p, n, [&](float v) {
+// Smallest key of p[0, n) past lo, at most `above`.
+template <bool VEC, int U, class K>
+__device__ uint64_t block_min_past(const float* __restrict__ p, int n, uint64_t lo, uint64_t above, const K& kf,
+                                   SelShared& sh) {
+  uint64_t mn = above;
+  each_value<VEC, MT, U>(p, n, [&](float v) {
     const uint64_t key = kf(v);
-    if (key > *lo && key < mn) mn = key;
+    if (key > lo && key < mn) mn = key;
   });
-  block_minmax(mn, mx, sh);
-  *hi = mn;
+  uint64_t none = 0;
+  block_minmax(mn, none, sh);
+  return mn;
 }
 
-// The two middle keys of a whole plane (equal for an odd count).
-template <bool VEC, class K>
+// The two middle keys of a whole plane (equal for an odd count), keys of W bits.
+template <bool VEC, int U, int W, class K>
 __device__ void block_middle(const float* __restrict__ p, int n, const K& kf, SelShared& sh, uint64_t* lo,
                              uint64_t* hi) {
-  uint64_t mn = ~0ull, mx = 0;
-  each_value<VEC, MT>(p, n, [&](float v) {
-    const uint64_t key = kf(v);
-    mn = key < mn ? key : mn;
-    mx = key > mx ? key : mx;
-  });
-  block_minmax(mn, mx, sh);
-  block_pair<VEC>(p, n, (uint32_t)((n - 1) / 2), !(n & 1), ~0ull, kf, mn, mx, sh, lo, hi);
+  uint32_t after = 0;
+  *lo = *hi = block_select<VEC, U, W>(p, n, (uint32_t)((n - 1) / 2), kf, W, 0, sh, &after);
+  if (!(n & 1) && after == 0) *hi = block_min_past<VEC, U>(p, n, *lo, ~0ull, kf, sh);
 }
 
 // Median of the values from its two middle keys.
@@ -242,29 +238,22 @@ __device__ __forceinline__ auto dev_key(double m) {
     return KeyDev64{m};
 }
 
-// Planes of at most MCAP elements: one block per plane, which reads its plane
-// once into LDS and selects there (LDSRC), and planes of any size where the
-// caller has no workspace: the block reads the plane once per pass.
-// The limit is what a selecting block holds in LDS; above it even two planes
-// are faster split.
+// One block per plane, which reads it once per pass: planes of at most MCAP elements
+// (their passes come from the caches, two blocks to a CU: 4096 planes of 4096 216 us;
+// a copy in LDS fills a CU with one block: 404), and planes of any size where the
+// caller has no workspace.
 constexpr int MCAP = 32768;  // values kept in LDS by a selecting block (128 KiB of the CU's 160)
 
-template <bool VEC, bool FP32, bool LDSRC>
-__global__ void __launch_bounds__(MT) k_band_mad(const float* __restrict__ planes, long long stride, int n,
+template <bool VEC, bool FP32, int U>
+__global__ void __launch_bounds__(MT, 8) k_band_mad(const float* __restrict__ planes, long long stride, int n,
                                                  double* __restrict__ mad) {
   __shared__ SelShared sh;
-  __shared__ float buf[LDSRC ? MCAP : 1];
   const float* p = planes + (size_t)blockIdx.x * (size_t)stride;
-  if constexpr (LDSRC) {
-    for (int i = threadIdx.x; i < n; i += MT) buf[i] = p[i];
-    __syncthreads();
-    p = buf;
-  }
   uint64_t a, b;
-  block_middle<VEC>(p, n, KeyValue{}, sh, &a, &b);
+  block_middle<VEC, U, KeyValue::W>(p, n, KeyValue{}, sh, &a, &b);
   const double m = value_median<FP32>(a, b, n);
-  __syncthreads();
-  block_middle<VEC>(p, n, dev_key<FP32>(m), sh, &a, &b);
+  const auto dev = dev_key<FP32>(m);
+  block_middle<VEC, U, decltype(dev)::W>(p, n, dev, sh, &a, &b);
   if (threadIdx.x == 0) mad[blockIdx.x] = dev_mad<FP32>(a, b, n);
 }
 
@@ -334,6 +323,7 @@ struct MadPlanes {
 // The 32-bit binning key of a stage, and the exact key its order refines to.
 template <int STAGE, bool FP32>
 struct MadKey {
+  static constexpr int W = STAGE && !FP32 ? 64 : 32;
   double m;
   __device__ uint64_t exact(float v) const {
     if constexpr (STAGE == 0) return KeyValue{}(v);
@@ -401,7 +391,7 @@ __global__ void __launch_bounds__(ST) k_mad_hist(MadPlanes io) {
   for (int i = threadIdx.x; i < NB; i += ST) hist[i] = 0;
   __syncthreads();
   const int at = blockIdx.x * SCHUNK;
-  each_value<VEC, ST>(io.p + (size_t)blockIdx.y * io.stride + at, min(SCHUNK, io.n - at), [&](float v) {
+  each_value<VEC, ST, 4>(io.p + (size_t)blockIdx.y * io.stride + at, min(SCHUNK, io.n - at), [&](float v) {
     const uint32_t key = kf.bin(v);
     if constexpr (SECOND) {
       if (key >> (32 - HBITS) == prefix) atomicAdd(&hist[(key >> (32 - HBITS - H2BITS)) & (H2BINS - 1)], 1u);
@@ -468,7 +458,7 @@ __global__ void __launch_bounds__(ST) k_mad_gather(MadPlanes io) {
   const int at = blockIdx.x * GCHUNK;
   uint64_t above = ~0ull;
   uint32_t abin = ~0u;  // binning key of `above`: exact keys are made only for values not past it
-  each_value<VEC, ST>(io.p + (size_t)blockIdx.y * io.stride + at, min(GCHUNK, io.n - at), [&](float v) {
+  each_value<VEC, ST, 4>(io.p + (size_t)blockIdx.y * io.stride + at, min(GCHUNK, io.n - at), [&](float v) {
     const uint32_t bin = kf.bin(v), b = bin >> shift;
     if (b > prefix) {
       if (bin > abin) return;
@@ -505,9 +495,10 @@ __global__ void __launch_bounds__(MT) k_mad_select(MadPlanes io, double* __restr
   const auto exact = [&](float v) { return kf.exact(v); };
   const uint32_t nc = st->ncand;
   const bool two = !(io.n & 1);
-  uint64_t a, b, mn = ~0ull, mx = 0;
+  uint64_t a, b;
   if (nc <= (uint32_t)MCAP) {
     const float* c = io.cand + (size_t)blockIdx.x * MCAP;
+    uint64_t mn = ~0ull, mx = 0;
     for (uint32_t i = threadIdx.x; i < nc; i += MT) {
       const float v = c[i];
       const uint64_t key = exact(v);
@@ -516,7 +507,7 @@ __global__ void __launch_bounds__(MT) k_mad_select(MadPlanes io, double* __restr
       mx = key > mx ? key : mx;
     }
     block_minmax(mn, mx, sh);
-    // the smallest key above the bin, used if the rank is the bin's last
+    // the smallest key past the bin, used if the rank is the bin's last
     uint64_t above = ~0ull, none = 0;
     if (two && st->rank2 + 1 == nc) {
       for (int i = threadIdx.x; i < io.gg; i += MT) {
@@ -525,9 +516,13 @@ __global__ void __launch_bounds__(MT) k_mad_select(MadPlanes io, double* __restr
       }
       block_minmax(above, none, sh);
     }
-    block_pair<false>(buf, (int)nc, st->rank2, two, above, exact, mn, mx, sh, &a, &b);
+    // the candidates' keys lie in [mn, mx]: only the bits in which these differ are open
+    const int top = mn == mx ? 0 : 64 - __clzll((long long)(mn ^ mx));
+    uint32_t after = 0;
+    a = b = block_select<false, 4, 0>(buf, (int)nc, st->rank2, exact, top, top == 64 ? 0 : mn & (~0ull << top), sh, &after);
+    if (two && after == 0) b = block_min_past<false, 4>(buf, (int)nc, a, above, exact, sh);
   } else {
-    block_middle<VEC>(io.p + (size_t)blockIdx.x * io.stride, io.n, exact, sh, &a, &b);
+    block_middle<VEC, 4, MadKey<STAGE, FP32>::W>(io.p + (size_t)blockIdx.x * io.stride, io.n, exact, sh, &a, &b);
   }
   if (threadIdx.x == 0) {
     if constexpr (STAGE == 0)
@@ -567,11 +562,11 @@ void launch_mad_stage(const MadPlanes& io, int nplanes, double* mad, hipStream_t
 template <bool VEC, bool FP32>
 void launch_mad(const float* planes, long long stride, int n, int nplanes, double* mad, void* work, hipStream_t s) {
   if (n <= MCAP) {
-    hipLaunchKernelGGL((k_band_mad<false, FP32, true>), dim3(nplanes), dim3(MT), 0, s, planes, stride, n, mad);
+    hipLaunchKernelGGL((k_band_mad<VEC, FP32, 1>), dim3(nplanes), dim3(MT), 0, s, planes, stride, n, mad);
     return;
   }
   if (!work) {
-    hipLaunchKernelGGL((k_band_mad<VEC, FP32, false>), dim3(nplanes), dim3(MT), 0, s, planes, stride, n, mad);
+    hipLaunchKernelGGL((k_band_mad<VEC, FP32, 4>), dim3(nplanes), dim3(MT), 0, s, planes, stride, n, mad);
     return;
   }
   // grid.y holds at most 65535 planes

@@ -159,27 +159,41 @@ def test_band_mad_split_planes(gpu, n, kind):
         assert np.array_equal(got, want), (arith, got, want)
 
 
+def _best_ms(api, x, reps=20):
+    api.band_mad_cuda(x)
+    ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+    best = float("inf")
+    for _ in range(reps):
+        ev[0].record()
+        api.band_mad_cuda(x)
+        ev[1].record()
+        torch.cuda.synchronize()
+        best = min(best, ev[0].elapsed_time(ev[1]))
+    return best
+
+
 def test_band_mad_time_is_linear_in_the_plane(gpu):
     """One plane of normal values, whose middle bin needs the second histogram,
     four times as large: about four times the time (every pass is linear),
     where a sum over the plane's histograms in every block made it eleven."""
     from shearcuda_amd import api
     gen = torch.Generator("cuda").manual_seed(3)
-    ms = {}
-    for e in (24, 26):
-        x = torch.randn(1, 1 << e, device="cuda", generator=gen)
-        api.band_mad_cuda(x)
-        ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
-        best = float("inf")
-        for _ in range(10):
-            ev[0].record()
-            api.band_mad_cuda(x)
-            ev[1].record()
-            torch.cuda.synchronize()
-            best = min(best, ev[0].elapsed_time(ev[1]))
-        ms[e] = best
+    ms = {e: _best_ms(api, torch.randn(1, 1 << e, device="cuda", generator=gen), 10) for e in (24, 26)}
     print("MAD of 2^24 and 2^26 elements: %.3f and %.3f ms" % (ms[24], ms[26]), flush=True)
     assert ms[26] < 7 * ms[24]
+
+
+def test_band_mad_small_planes_two_blocks_to_a_cu(gpu):
+    """1, 8 and 16 planes of 4096 for every CU: with room for two blocks on a CU
+    a further plane for every CU takes about half of what the first takes (0.43
+    to 0.52 measured); a block that fills its CU (a copy of the plane in LDS)
+    took 0.74 to 0.86."""
+    from shearcuda_amd import api
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    gen = torch.Generator("cuda").manual_seed(4)
+    t = {k: _best_ms(api, torch.randn(k * cus, 4096, device="cuda", generator=gen), 40) for k in (1, 8, 16)}
+    print("MAD of 1, 8, 16 planes of 4096 per CU: %s ms" % t, flush=True)
+    assert t[16] - t[8] < 0.65 * 8 * t[1]
 
 
 @pytest.mark.parametrize("nplanes,n", [(2, 262144), (2, 262145), (1, 1 << 20), (3, 1 << 20)])
