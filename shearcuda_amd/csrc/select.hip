@@ -558,6 +558,25 @@ void launch_mad_stage(const MadPlanes& io, int nplanes, double* mad, hipStream_t
   hipLaunchKernelGGL((k_mad_select<STAGE, VEC, FP32>), dim3(nplanes), dim3(MT), 0, s, io, mad);
 }
 
+// Whether a call with a workspace splits its planes over blocks or gives each to one,
+// where many planes fill the chip by themselves.  Split / one block, us, 33000 elements:
+//   FP32  1 plane 43 / 33, 49 planes 48 / 34, 512 109 / 69, 2048 366 / 262
+//   FP64  1 plane 47 / 57, 49 planes 52 / 58, 512 118 / 111, 1100 235 / 273, 2048
+//         399 / 418, 8192 2141 / 2278, 16384 3224 / 3039
+// 65536 elements:
+//   FP32  49 planes 50 / 53, 128 63 / 54, 384 122 / 115, 512 146 / 146, 1024 269 / 297
+//   FP64  128 planes 68 / 98, 2048 624 / 847
+// and 131072 elements: FP32 128 planes 86 / 102.  One block per plane for FP32 below
+// 49152 elements, and up to 98304 for 65 to 511 planes; for FP64 below 49152 elements
+// and more than 4096 planes (there it spares the workspace).
+constexpr int SPLIT_N = 49152, SPLIT_PLANES = 4096;
+template <bool FP32>
+bool split_pays(int n, int nplanes) {
+  if (n <= MCAP) return false;
+  if (FP32) return n >= 2 * SPLIT_N || (n >= SPLIT_N && (nplanes <= 64 || nplanes >= 512));
+  return n >= SPLIT_N || nplanes <= SPLIT_PLANES;
+}
+
 // VEC: float4 loads, for planes that all start on 16 bytes.
 template <bool VEC, bool FP32>
 void launch_mad(const float* planes, long long stride, int n, int nplanes, double* mad, void* work, hipStream_t s) {
@@ -565,7 +584,7 @@ void launch_mad(const float* planes, long long stride, int n, int nplanes, doubl
     hipLaunchKernelGGL((k_band_mad<VEC, FP32, 1>), dim3(nplanes), dim3(MT), 0, s, planes, stride, n, mad);
     return;
   }
-  if (!work) {
+  if (!work || !split_pays<FP32>(n, nplanes)) {
     hipLaunchKernelGGL((k_band_mad<VEC, FP32, 4>), dim3(nplanes), dim3(MT), 0, s, planes, stride, n, mad);
     return;
   }

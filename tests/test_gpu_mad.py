@@ -234,3 +234,17 @@ def test_band_mad_of_the_largest_plane(gpu):
     want = int(np.searchsorted(np.cumsum(dev), mid, side="right")) / 0.6745
     print("case largest plane", flush=True)
     assert float(api.band_mad_cuda(t, "fp32")[0]) == want
+
+
+@pytest.mark.parametrize("nplanes,n", [(64, 49151), (64, 49152), (65, 49152), (65, 98303), (65, 98304), (511, 49152),
+                                       (512, 49152), (4096, 32769), (4097, 32769)])
+def test_band_mad_around_the_split_rule(gpu, nplanes, n):
+    """Plane counts and sizes on both sides of the rule that splits planes over
+    blocks: every tenth plane and the last against numpy."""
+    from shearcuda_amd import api
+    a = np.random.default_rng(n + nplanes).standard_normal((nplanes, n), dtype=np.float32)
+    t = torch.from_numpy(a).cuda()
+    some = sorted(set(range(0, nplanes, max(1, nplanes // 10))) | {nplanes - 1})
+    for arith, ref in (("fp64", _mad64), ("fp32", _mad32)):
+        got = api.band_mad_cuda(t, arith).cpu().numpy()[some]
+        assert np.array_equal(got, np.array([ref(a[i]) for i in some])), arith
