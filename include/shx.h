@@ -353,8 +353,9 @@ int shx_band_mad(const float* planes, long long plane_elems, long long plane_str
 
 /* shx_band_mad with a device workspace of at least
  * shx_band_mad_workspace(plane_elems, nplanes) bytes (16-byte aligned; NULL
- * or 0 bytes where that is 0), over which planes of more than 32768 elements
- * are split over many workgroups instead of one each.  Same results. */
+ * or 0 bytes where that is 0), over which large planes are split over many
+ * workgroups instead of one each.  At most 268 MB and an eighth of 2048
+ * planes: the planes of a larger stack take turns.  Same results. */
 size_t shx_band_mad_workspace(long long plane_elems, int nplanes);
 int shx_band_mad_ws(const float* planes, long long plane_elems, long long plane_stride, int nplanes, int arith,
                     double* mad, void* work, size_t work_bytes, void* stream);

@@ -83,3 +83,20 @@ def test_band_thresholds_match_nsst_HT():
             band_thresholds(D, 10.0, bad, (0.0, 3.0, 4.0))
     with pytest.raises(ValueError):
         band_thresholds(D, 10.0, sc, (0.0, 3.0))
+
+
+def test_median_workspace_is_bounded():
+    """The workspace of the split medians: none for planes one block takes, 128 KB
+    and about an eighth of its bytes for a plane, and never more than 2048 planes'
+    (a larger stack goes through in groups)."""
+    from shearcuda_amd import _lib
+    ws = _lib.lib.shx_band_mad_workspace
+    assert ws(32768, 49) == 0 and ws(262144, 0) == 0 and ws(1 << 31, 1) == 0
+    one = ws(262144, 1)
+    assert 131072 + 262144 // 2 <= one <= 131072 + 262144 // 2 + 1024
+    assert ws(262144, 49) == 49 * one and ws(262144, 2048) == 2048 * one
+    assert ws(32769, 1000) > 0
+    for n in (32769, 40000, 65536, 262144):
+        for planes in (2049, 3000, 4096, 4097, 100000, (1 << 31) - 1):
+            assert ws(n, planes) <= 2048 * (131072 + n // 2 + 16384), (n, planes)
+    assert ws((1 << 31) - 1, 1) < (1 << 30) + (1 << 22)

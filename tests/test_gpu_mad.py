@@ -248,3 +248,21 @@ def test_band_mad_around_the_split_rule(gpu, nplanes, n):
     for arith, ref in (("fp64", _mad64), ("fp32", _mad32)):
         got = api.band_mad_cuda(t, arith).cpu().numpy()[some]
         assert np.array_equal(got, np.array([ref(a[i]) for i in some])), arith
+
+
+def test_band_mad_in_groups(gpu):
+    """More planes than go through the split passes together (2048), the groups
+    after the first in the workspace of the ones before: every plane the same
+    whichever group it falls in, a few against numpy."""
+    from shearcuda_amd import api
+    n, nplanes = 49155, 2051
+    a = np.random.default_rng(8).standard_normal((7, n), dtype=np.float32)
+    t = torch.from_numpy(a).cuda().repeat(293, 1)
+    assert t.shape[0] == nplanes
+    t[5::7] *= torch.arange(1, 294, device="cuda", dtype=torch.float32)[:, None]
+    for arith, ref in (("fp64", _mad64), ("fp32", _mad32)):
+        got = api.band_mad_cuda(t, arith).cpu().numpy()
+        for k in (0, 1, 2, 3, 4, 6):
+            assert np.all(got[k::7] == ref(a[k])), (arith, k)
+        for i in (5, 5 + 7 * 146, 5 + 7 * 292):
+            assert got[i] == ref(t[i].cpu().numpy()), (arith, i)
