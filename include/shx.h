@@ -295,7 +295,8 @@ int shx_mirdwt_adjoint(const float* x_bar, int m, int n, const double* h, int lh
 
 /* Soft-thresholded synthesis and its backward, with the thresholds applied inside
  * the level kernels; available where shx_rdwt_fused(n, L, lh) is 1 (filters of at
- * most 8 taps, rows of at most 512 or dilated filters of at most 256 columns).
+ * most 8 taps, rows of at most 512 or dilated filters of at most 256 columns;
+ * 0 for arguments that shx_mrdwt refuses).
  * th_dev: 1 + 3 L thresholds (yl, then [lh hl hh] per level), shared by the images.
  * shx_mirdwt_soft: x = mirdwt(soft(yl), soft(yh)); work: 2*m*n*nimg floats.
  * shx_wave_shrink_mask: with (c_l, c_h) = mrdwt(b) and the output gradient g,

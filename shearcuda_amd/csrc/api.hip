@@ -2279,7 +2279,10 @@ int shx_mirdwt_adjoint(const float* x_bar, int m, int n, const double* h, int lh
                   [&](float* t) { return shx::rdwt_analysis(x_bar, yl_bar, yh_bar, t, m, n, L, f, nimg, s); });
 }
 
-int shx_rdwt_fused(int n, int L, int lh) { return shx::rdwt_fused(n, L, lh) ? 1 : 0; }
+int shx_rdwt_fused(int n, int L, int lh) {
+  // 0 for what rdwt_check refuses (its shifts assume valid levels)
+  return n >= 1 && L >= 1 && L <= 12 && lh >= 2 && shx::rdwt_fused(n, L, lh) ? 1 : 0;
+}
 
 int shx_mirdwt_soft(const float* yl, const float* yh, int m, int n, const double* h, int lh, int L,
                     const float* th_dev, float* x, float* work, int nimg, void* stream) {

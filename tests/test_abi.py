@@ -100,3 +100,14 @@ def test_median_workspace_is_bounded():
         for planes in (2049, 3000, 4096, 4097, 100000, (1 << 31) - 1):
             assert ws(n, planes) <= 2048 * (131072 + n // 2 + 16384), (n, planes)
     assert ws((1 << 31) - 1, 1) < (1 << 30) + (1 << 22)
+
+
+@pytest.mark.parametrize("n,L,lh,fused", [(512, 9, 8, 1), (513, 1, 8, 1), (1024, 6, 8, 1), (1024, 7, 8, 0), (4096, 12, 2, 0),
+                                          (1024, 3, 10, 0), (1024, 3, 7, 0), (512, 0, 4, 0), (1024, 0, 4, 0),
+                                          (1024, 13, 4, 0), (1024, 33, 4, 0), (1024, 40, 4, 0), (1024, -1, 4, 0),
+                                          (1024, 3, 0, 0), (1024, 3, -2, 0), (0, 3, 4, 0), (-8, 3, 4, 0)])
+def test_rdwt_fused_answers_for_any_arguments(n, L, lh, fused):
+    """Which transforms run fused levels; 0 for levels, taps and rows that the
+    transforms themselves refuse, whatever their value."""
+    from shearcuda_amd import _lib
+    assert _lib.lib.shx_rdwt_fused(n, L, lh) == fused
