@@ -266,7 +266,7 @@ def test_identity_and_lowpass_at_128(mods):
 @pytest.mark.parametrize("n,group,dirs,mode", [(32, 1, (4, 3, 2), 1), (48, 3, (4, 3, 2), 1.5), (64, 5, (4, 2, 2), 1),
                                                (64, 8, (3, 2, 2), 2), (128, 7, (3, 2, 2), 1)])
 def test_slab_band_loop_equals_bands(mods, n, group, dirs, mode):
-    """The band loop that keeps a slab in LDS (every FFT grid it covers, groups
+    """The band loop that keeps a slab in LDS (FFT grids 32, 48, 64, 80 and 144, groups
     that do not divide the band count, more splits than bands left in a group)
     against the materialised bands, thresholded and summed; thresholds lie in
     a gap of each band's magnitudes."""
@@ -302,7 +302,7 @@ def test_slab_band_loop_equals_bands(mods, n, group, dirs, mode):
                                                (128, (2, 2, 2), 1, 6)])
 def test_analysis_adjoint_at_ragged_groups(mods, n, dirs, mode, group):
     """The adjoint sums a group's bands in four chunks: groups that leave
-    chunks empty or uneven, on every FFT grid, against the adjoint identity
+    chunks empty or uneven, on grids of 32 to 144, against the adjoint identity
     and the group of 8.  The groups only reorder a sum of FP32 products, so
     both share the identity's tolerance."""
     print("case adjoint groups n=%d group=%d" % (n, group), flush=True)
@@ -354,4 +354,41 @@ def test_analysis_adjoint_one_band_per_group(mods, n, dirs, mode):
     ref = wide.analysis_adjoint(y)[:, :nlev].double()
     assert float((got.double() - ref).abs().max() / ref.abs().max()) < TOL
     wide.close()
+    sh.close()
+
+
+@pytest.mark.parametrize("group", [1, 5])
+def test_smallest_fft_grid(mods, group):
+    """The 24^3 grid of a level of side 8: bands against the oracle, the slab
+    band loop against the thresholded bands, the transpose by its identity."""
+    print("case grid 24 group=%d" % group, flush=True)
+    dirs, nvol = (2,), 2
+    F = o3.meyer_filters_3d([2])
+    sh = mods[1].Shear3D(8, dirs, 1)
+    assert sh.sides == [8, 8] and sh.fft_sides == [24]
+    plan = mods[1].Plan3D(sh, nvol, group=group)
+    rng = np.random.default_rng(24)
+    s = rng.standard_normal((nvol, sh.subs_elems)) * 20
+    st = torch.tensor(s, dtype=torch.float32, device="cuda")
+    bands = plan.analysis(st)
+    b = sh.split_bands(bands)[0]
+    th = torch.empty(nvol, sh.nbands, device="cuda")
+    for v in range(nvol):
+        conv = o3._SameConv(s[v, :512].reshape(8, 8, 8), (24, 24, 24))
+        for k, f in enumerate(o3.band_list(F, 0)):
+            want = conv(f)
+            assert _rel(b[v, k].cpu().numpy(), want) < TOL, (v, k)
+            a = torch.sort(b[v, k].abs().reshape(-1)).values[128:385]
+            i = int(torch.argmax(a[1:] - a[:-1]))
+            th[v, k] = 0.5 * (a[i] + a[i + 1])
+    want = torch.where(b.abs() > th[:, :, None, None, None], b, torch.zeros_like(b)).double().sum(1)
+    got = sh.split_subs(plan.dec_thresh_rec(st, th))[0].double()
+    assert float((got - want).abs().max() / want.abs().max()) < TOL
+    y = torch.tensor(rng.standard_normal((nvol, sh.bands_elems)), dtype=torch.float32, device="cuda")
+    aty = plan.analysis_adjoint(y)[:, :512].double()
+    for v in range(nvol):
+        lhs = float(torch.dot(bands[v].double(), y[v].double()))
+        rhs = float(torch.dot(st[v, :512].double(), aty[v]))
+        assert abs(lhs - rhs) < TOL * float(bands[v].double().norm() * y[v].double().norm())
+    plan.close()
     sh.close()

@@ -156,3 +156,80 @@ def test_fused_wave_shrink_equals_separate_calls(gpu, shape, levels, name):
     assert torch.equal(out.detach(), want)
     assert torch.equal(gb, gw)
     assert float((gt - gth).abs().max()) <= 1e-5 * float(g.abs().sum())
+
+
+@pytest.mark.parametrize("nimg,m,n,levels,name", [(210, 72, 24, 2, "Daubechies"), (256, 24, 520, 1, "Symmlet"),
+                                                  (128, 68, 40, 2, "Haar")])
+def test_fused_wave_shrink_strips_of_16_and_8_rows(gpu, nimg, m, n, levels, name):
+    """Large batches take strips of 16 and 8 rows in the thresholded level
+    kernels: the same bits as the same images in batches of four (strips of 4
+    rows), threshold gradients to the rounding of a sum over the images."""
+    from shearcuda_amd import separation
+    from shearcuda_amd.wavelets import MakeONFilter
+    h = MakeONFilter(name, 4)
+    gen = torch.Generator("cuda").manual_seed(nimg)
+    b = torch.randn(nimg, m, n, device="cuda", generator=gen) * 20
+    g0 = torch.randn(nimg, m, n, device="cuda", generator=gen)
+    th = torch.linspace(2.0, 15.0, 1 + 3 * levels, device="cuda")
+
+    def run(s):
+        bb, tt = b[s].clone().requires_grad_(True), th.clone().requires_grad_(True)
+        out = separation.WaveShrink.apply(bb, tt, h, levels)
+        return (out.detach(),) + torch.autograd.grad(out, [bb, tt], g0[s].contiguous())
+    out, gb, gt = run(slice(0, nimg))
+    total = torch.zeros_like(gt, dtype=torch.float64)
+    for i in range(0, nimg, 4):
+        s = slice(i, min(nimg, i + 4))
+        o4, b4, t4 = run(s)
+        assert torch.equal(o4, out[s]) and torch.equal(b4, gb[s])
+        total += t4.double()
+    assert float((gt.double() - total).abs().max()) <= 1e-5 * float(g0.abs().sum())
+
+
+@pytest.mark.parametrize("taps,shape,levels", [(10, (24, 40), 2), (32, (64, 64), 1), (8, (128, 1024), 7)])
+def test_wave_shrink_separate_passes_against_oracle(gpu, taps, shape, levels):
+    """WaveShrink where the levels run as separate passes (long filters, deep
+    levels of long rows), forward and both gradients against the oracle's
+    transforms in FP64; each threshold lies in the widest gap of the middle
+    half of its band's magnitudes, so FP32 makes the same decisions."""
+    from shearcuda_amd import separation
+    from shearcuda_amd._lib import lib
+    m, n = shape
+    assert lib.shx_rdwt_fused(n, levels, taps) == 0
+    rng = np.random.default_rng(taps)
+    h = rng.standard_normal(taps)
+    h /= np.linalg.norm(h)
+    b = (rng.standard_normal((1, m, n)) * 20).astype(np.float32)
+    gr = rng.standard_normal((1, m, n)).astype(np.float32)
+    yl, yh = w.mrdwt(b[0], h, levels)
+    bands = [yl] + [yh[:, k * n:(k + 1) * n] for k in range(3 * levels)]
+    th = []
+    for c in bands:
+        a = np.sort(np.abs(c).ravel())
+        a = a[a.size // 4:3 * a.size // 4 + 2]
+        i = int(np.argmax(np.diff(a)))
+        th.append(0.5 * (a[i] + a[i + 1]))
+    th = np.float32(th)
+    keep = [np.abs(c) > t for c, t in zip(bands, th)]
+
+    def syn(cs):
+        return w.mirdwt(cs[0], np.concatenate(cs[1:], axis=1), h, levels)
+    want = syn([np.where(k, c - np.sign(c) * t, 0.0) for c, k, t in zip(bands, keep, th.astype(np.float64))])
+    bb, tt = g(b).requires_grad_(True), g(th).requires_grad_(True)
+    out = separation.WaveShrink.apply(bb, tt, h, levels)
+    gb, gt = torch.autograd.grad(out, [bb, tt], g(gr))
+    assert np.abs(out[0].detach().cpu().numpy() - want).max() < 1e-5 * np.abs(want).max()
+    # the gradient of <out, gr> along v is <syn(mask . bands of v), gr>
+    gb = gb[0].cpu().numpy().astype(np.float64)
+    for _ in range(3):
+        v = rng.standard_normal((m, n))
+        vl, vh = w.mrdwt(v, h, levels)
+        vb = [vl] + [vh[:, k * n:(k + 1) * n] for k in range(3 * levels)]
+        ref = np.sum(syn([np.where(k, c, 0.0) for c, k in zip(vb, keep)]) * gr[0])
+        assert abs(np.sum(gb * v) - ref) < 1e-5 * np.linalg.norm(gb) * np.linalg.norm(v)
+    zero = [np.zeros((m, n)) for _ in bands]
+    for k in range(len(bands)):
+        cs = list(zero)
+        cs[k] = np.where(keep[k], -np.sign(bands[k]), 0.0)
+        s = syn(cs)
+        assert abs(float(gt[k]) - np.sum(s * gr[0])) < 1e-5 * np.linalg.norm(s) * np.linalg.norm(gr), k
