@@ -545,13 +545,14 @@ __global__ void __launch_bounds__(MT) k_mad_select(MadPlanes io, double* __restr
 
 // Whether the gather's blocks each add up the plane's second histograms (gh of 4 KB).
 // A launch of k_mad_find instead costs 2-3 us, also where no plane needs the second
-// histogram (up to 512^2: 49 planes 91 us); the sums of all blocks grow with the
-// square of a plane's size.  In the gather for planes of up to 512^2 and while all
-// sums are at most 64 MB (one 1024^2 plane 68 us, with the launch 72); beyond, the
-// launch: 49 x 1024^2 282 -> 220 us, 192 x 128^3 2964 -> 1670, 2^27 elements 31.6 ->
-// 3.9 ms.
+// histogram; the sums of all blocks grow with the square of a plane's size.  In the
+// gather / by a launch, us: 49 normal planes of 400000 115 / 118, of 800000 180 / 182,
+// of 1024^2 (which need it) 280 / 217; one plane of 128^3 91 / 94, four 121 / 109, 192
+// 2964 / 1670; 2^27 elements 31.6 / 3.9 ms.  In the gather for planes of up to 50
+// histograms (819200 elements, from where normal planes begin to need them) and while
+// all sums are at most 128 MB.
 bool find2_in_gather(const MadPlanes& io, int nplanes) {
-  return io.gh <= 16 || (long long)io.gh * io.gg * nplanes <= 16384;
+  return io.gh <= 50 || (long long)io.gh * io.gg * nplanes <= 32768;
 }
 
 template <int STAGE, bool VEC, bool FP32>

@@ -196,7 +196,7 @@ def test_band_mad_small_planes_two_blocks_to_a_cu(gpu):
     assert t[16] - t[8] < 0.65 * 8 * t[1]
 
 
-@pytest.mark.parametrize("nplanes,n", [(2, 262144), (2, 262145), (1, 1 << 20), (3, 1 << 20)])
+@pytest.mark.parametrize("nplanes,n", [(2, 262145), (8, 819200), (8, 819201), (4, 1 << 20), (5, 1 << 20)])
 @pytest.mark.parametrize("kind", ["offset", "normal"])
 def test_band_mad_second_bin_forms(gpu, nplanes, n, kind):
     """Both places that find the bin of the second histogram (a launch of its
