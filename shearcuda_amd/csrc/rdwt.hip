@@ -120,9 +120,10 @@ __global__ void k_rdwt_rows_syn(const float* __restrict__ X, const float* __rest
 // rows (plus the taps' LH - 1 rows of warm-up) and the intermediate planes of
 // the separate passes, 4 planes of traffic per level, never reach memory.
 // The separate passes below read every tap from global memory behind an
-// integer remainder: 315 and 363 us for the 3-level analysis and synthesis of
-// 4 x 1000 x 1496 with 8 taps against 80 and 110 us here, 3.3 and 2.4 TB/s of
-// the values that have to move (the level's rows, bound by loads in flight).
+// integer remainder: calls of 295 and 345 us for the 3-level analysis and synthesis
+// of 4 x 1000 x 1496 with 8 taps against 80 and 100 us here, 3.3 and 2.6 TB/s of
+// the values that have to move (the transform's input and bands; bound by loads in
+// flight).
 struct RdwtLevel {
   const float* in;   // low band of the level (analysis: its input)
   float* out;        // analysis: next low band; synthesis: result
@@ -220,7 +221,7 @@ __global__ void __launch_bounds__(RT) k_rdwt_level_an(RdwtLevel a, RdwtTaps<LH> 
 }
 
 // SOFT: the bands are soft-thresholded as they are read (8 x 512^2, 3 levels,
-// 4 taps: 38 us; with a pass of its own over the bands 88).
+// 4 taps: 38 us of kernels; with a pass of its own over the bands 88).
 template <int LH, int K, bool SOFT>
 __global__ void __launch_bounds__(RT) k_rdwt_level_syn(RdwtLevel a, RdwtTaps<LH> f) {
   __shared__ float lu[2][4][RT], lv[2][4][RT];
@@ -306,7 +307,7 @@ __global__ void __launch_bounds__(RT) k_rdwt_level_syn(RdwtLevel a, RdwtTaps<LH>
 //   bands of g * 1[|bands of b| > t] to yh, gth += sum -sign(b) 1[|b| > t] g,
 // and the low bands of both on (of g masked at the last level).  The bands of b are
 // never stored; separate passes wrote both stacks and read them back for the mask
-// (8 x 512^2, 3 levels, 4 taps: 164 us against 68).
+// (8 x 512^2, 3 levels, 4 taps: 164 us of kernels against 68).
 template <int LH, int K>
 __global__ void __launch_bounds__(RT) k_rdwt_level_mask(RdwtLevel a, RdwtTaps<LH> f, RdwtTaps<LH> f2) {
   __shared__ float lb[2][4][2][RT], lg[2][4][2][RT];

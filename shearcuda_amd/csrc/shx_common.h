@@ -54,8 +54,8 @@ __host__ __device__ constexpr int ilog2(int n) { return n <= 1 ? 0 : 1 + ilog2(n
 // Non-temporal accesses: for data that crosses memory once between two kernels
 // (band spectra, coefficients), so that it does not push out of the L2 what a
 // kernel's blocks share (scale spectra, filter spectra, twiddles).  With the band
-// spectra of a 2D plan accessed so, the kernels of a denoise went from 115 to 111
-// us (512^2), 922 to 877 (48 x 256^2) and 2400 to 2290 (8 x 1024^2).
+// spectra of a 2D plan accessed so, a denoise went from 819 to 795 us (48 x 256^2)
+// and from 2228 to 2108 (8 x 1024^2), a 512^2 step from 123 to 115.
 __device__ __forceinline__ float2 load_nt(const float2* p) {
   using V = __attribute__((ext_vector_type(2))) float;
   const V v = __builtin_nontemporal_load(reinterpret_cast<const V*>(p));

@@ -633,9 +633,7 @@ __global__ void __launch_bounds__(RowCfg<L>::T) k_rows_c2r_mask_r2c(PlaneSet Tin
 // R1 x R2.  T = CT * R2 threads; element (u, c) of the LDS tile is linear
 // element u*CT + c.
 // Column tile widths: 8; 16 where the tile fits the LDS (L <= 512); 4 where
-// a block still fills a wave (4 R2 >= 64).  Narrow tiles use a quarter of
-// each 128-byte row line; the XCD-aware block order keeps the neighbouring
-// tiles that share a line in one L2.
+// a block still fills a wave (4 R2 >= 64).
 template <int L>
 struct ColTile {
   static constexpr bool wide = L / 2 >= 16 && L <= 512;
@@ -1021,23 +1019,23 @@ __device__ __forceinline__ void col_block_order(int& tile, int& plane, int& img,
 }
 
 // Block order of the decomposition column passes (and of the reconstruction
-// passes up to 512^2), after the same XCD remap:
-// the TG column tiles that share a 128-byte line (TG = 16 / CT for tiles of
-// CT complex columns) fastest, then the image, then the plane (band slot),
-// then the tile group.  An XCD then runs every band of a few neighbouring
-// tiles back to back, so the scale spectrum tile (read by all bands of its
-// scale), each filter tile (read by the bands sharing it and by every image
-// of a batch) come from its L2 after the first read, and each line is fetched
-// once for the TG tiles that share it (row-major spectra only; in strips of four
-// columns a tile's lines are its own, and the figures here are from before the
-// strips).  Measured against the tile-fastest
-// order of the other column passes: 512^2, 8 columns, 28.8 -> 24.8 us
-// (counted fetch 66 -> 47 MB); 1024^2, 8 columns, 91 -> 86 us; with the image
-// after the tile group instead of before the plane, the batched mix ran 1.5%
-// slower.  The reconstruction (planes = direction groups) shares only filter
-// tiles; it takes this order for one image up to 512^2 (three-pass 4-column
-// pass 29.3 -> 26.9 us) and the tile-fastest order for batches and at
-// 1024^2, where it measured faster.
+// passes up to 512^2), after the same XCD remap: TG neighbouring column tiles
+// fastest, then the image, then the plane (band slot), then the tile group.  An
+// XCD then runs every band of a few neighbouring tiles back to back, so the scale
+// spectrum tile (read by all bands of its scale) and each filter tile (read by the
+// bands sharing it and by every image of a batch) come from its L2 after the first
+// read.  TG = 16 / CT tiles of CT columns shared a 128-byte line of row-major
+// spectra; in strips a tile's lines are its own.  Against the tile-fastest order of
+// the other column passes (image-only denoise, graph replays, DCT form on both
+// sides, us, this order / that):
+//   decomposition   512^2 112 / 113, 8 x 512^2 502 / 505, 1024^2 340 / 363, 8 x 1024^2
+//                   2165 / 2263, 8 x 256^2 162 / 166; but 256^2 75 / 73.5, 48 x 256^2
+//                   810 / 799
+//   reconstruction  of one image up to 512^2 (planes = direction groups, which share
+//                   only filter tiles): 512^2 112 / 116; but 256^2 75 / 73
+// and with TG = 1 in all of them 256^2 74.6, 8 x 256^2 159, 48 x 256^2 793, 512^2 110,
+// 8 x 512^2 494, 1024^2 339, 8 x 1024^2 2158.  The reconstruction of batches and at
+// 1024^2 takes the tile-fastest order (with row-major spectra 112 against 115 us).
 template <int TG>
 __device__ __forceinline__ void col_block_order_lines(int& tile, int& plane, int& img) {
   const int nt = gridDim.x, np = gridDim.y, ni = gridDim.z;
@@ -1133,9 +1131,9 @@ __global__ void __launch_bounds__(CT_ * Split<L>::R2) k_cols_rec(const float2* _
   __shared__ float2 buf[C::LDS];
   __shared__ float2 accl[ColRecAcc<L, CT_>::SIZE];
   int tile, slot, b;
-  // one image up to 512^2: the line-grouped order (measured 29.6 -> 28.4 us
-  // at 512^2, 4 columns); batches and 1024^2: tile fastest, then image (the
-  // images reading one filter tile together; 112 against 115 us at 1024^2)
+  // one image up to 512^2: the tile-grouped order (figures at
+  // col_block_order_lines); batches and 1024^2: tile fastest, then image (the
+  // images reading one filter tile together)
   if (L <= 512 && gridDim.z == 1)
     col_block_order_lines<(16 / C::CT > 1 ? 16 / C::CT : 1)>(tile, slot, b);
   else
@@ -1252,7 +1250,7 @@ __global__ void __launch_bounds__(CT * 64) k_cols_rec3(const float2* __restrict_
   constexpr int NH = L / 2, NV = G::NV;
   __shared__ float2 buf[E::LDS];
   int tile, slot, b;
-  if (gridDim.z == 1)  // one image: 29.3 -> 26.9 us at 4 columns
+  if (gridDim.z == 1)  // one image: a 512^2 denoise 112 us, 116 tile-fastest
     col_block_order_lines<(16 / CT > 1 ? 16 / CT : 1)>(tile, slot, b);
   else
     col_block_order(tile, slot, b, map.gshare);

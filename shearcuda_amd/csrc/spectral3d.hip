@@ -474,6 +474,9 @@ __global__ void __launch_bounds__(CT * Split<N>::R2) k3_pencil_inv(Pencil3Inv io
 // 8 bands of two 128^3 volumes: rows 82 -> 62 us (290 MB: the copy rate), columns
 // and pencils 67 + 50 -> 73 us (172 MB; the block's LDS and vector pipes are each
 // busy half of the time, one after the other: one block per CU).
+// The grid of 128 has no such split here: it belongs to levels of side 80 (or 64 with
+// filters of 40 and more), which no dictionary of the workloads has, so its two row
+// kernels and the separate passes serve it, as they do the grids of 8 and 16.
 template <int N>
 struct Split3;
 template <> struct Split3<24> { static constexpr int P = 4, Q = 6, NP = 12; };
