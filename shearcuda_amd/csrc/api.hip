@@ -870,7 +870,7 @@ void stages_denoise_dag(shx_dict* d, Work& w, int nimg, const float* x, long lon
     }
     Stage b{"cols_dec" + sfx, (1 + 2.0 * nb) * P, [=] {
               return shx::launch_cols_dec(L, Y1, w.s_spec / 2, T, w.s_band / 2, Hm, Hb, m, nimg, d->tw, sj, w.ct_dec,
-                                          true);
+                                          true, false, d->nbands);
             }};
     b.stream = sj;
     if (w.dct_front) b.waits = {made[j]};
@@ -880,7 +880,8 @@ void stages_denoise_dag(shx_dict* d, Work& w, int nimg, const float* x, long lon
     cc.stream = sj;
     st.push_back(cc);
     Stage e{"cols_rec" + sfx, (2.0 * nb + ng) * P, [=] {
-              return shx::launch_cols_rec(L, T, w.s_band / 2, Q, w.s_q / 2, Hm, Hb, m, nimg, d->tw, sj, w.ct_rec);
+              return shx::launch_cols_rec(L, T, w.s_band / 2, Q, w.s_q / 2, Hm, Hb, m, nimg, d->tw, sj, w.ct_rec,
+                                          d->nbands);
             }};
     e.stream = sj;
     if (w.dct_back) {  // the back end takes the partials of every scale at once

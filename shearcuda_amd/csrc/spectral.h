@@ -96,11 +96,12 @@ hipError_t launch_rows_c2r_mask_r2c(int L, const PlaneSet& Tin, const PlaneSet& 
                                     int nimg, const ThreshSpec& th, float* gth, const float2* tw, hipStream_t s);
 // ct: column tile width of the block (4, 8 or 16 where col_tile_ok; 0 = the
 // default for L).  pre: Y1 is already column-transformed (launch_cols_fwd).
-// rows: the plain inverse row pass (launch_rows_c2r) reads Tout next.
+// rows: the plain inverse row pass (launch_rows_c2r) reads Tout next.  beside: the
+// bands of the plan when this launch is one of its scales, which run side by side.
 bool col_tile_ok(int L, int ct);
 hipError_t launch_cols_dec(int L, const float2* Y1, long long y1_stride, float2* Tout, long long t_stride,
                            const float2* Hm, const float2* Hb, const BandMap& map, int nimg, const float2* tw,
-                           hipStream_t s, int ct = 0, bool pre = false, bool rows = false);
+                           hipStream_t s, int ct = 0, bool pre = false, bool rows = false, int beside = 0);
 // In-place forward column FFT of nplanes packed spectra (stride y1_stride per image).
 hipError_t launch_cols_fwd(int L, float2* Y1, long long y1_stride, int nplanes, int nimg, const float2* tw,
                            hipStream_t s, int ct = 0);
@@ -125,6 +126,6 @@ hipError_t launch_dct_rec(int L, int step, const float2* Qg, long long qs, const
                           hipStream_t s);
 hipError_t launch_cols_rec(int L, const float2* U, long long u_stride, float2* Q, long long q_stride,
                            const float2* Hm, const float2* Hb, const BandMap& map, int nimg, const float2* tw,
-                           hipStream_t s, int ct = 0);
+                           hipStream_t s, int ct = 0, int beside = 0);
 
 }  // namespace shx

@@ -1362,19 +1362,22 @@ struct Launch {
                        tw);
     return hipGetLastError();
   }
-  // Whether a column pass stores its spectra non-temporally (graph replays, us).
-  // 256^2: from 480 planes (120 MB) in one launch on.  Below that what follows reads
-  // them faster from the caches (8 images, denoise with coefficients 183 non-temporal,
-  // 175 not; 4 images, transform 62.3 and 60.8; a plan of one launch per scale, whose
-  // launches are a third as large: 16 images 434 and 406); above it they push out what
-  // the blocks share (16 images in one launch 341 and 359, 20 images 426 and 435).
+  // Whether a column pass stores its spectra non-temporally (us, graph replays but
+  // where said).  256^2: from 480 planes (120 MB) in one launch on.  Below that what
+  // follows reads them faster from the caches (8 images, denoise with coefficients 183
+  // non-temporal, 175 not; 4 images, transform 62.3 and 60.8); above it they push out
+  // what the blocks share (16 images 341 and 359, 20 images 426 and 435).  A plan whose
+  // scales run side by side (beside: its bands, else 0) holds its launches' planes
+  // apart in time: from 960 planes on (16 images 434 and 410, 20 images 516 and 496 but
+  // launched one by one 510 and 522, 48 images 925 and 952).
   // 512^2: always, but for one image whose planes go straight to the plain row pass
   // (rows: transform 80 non-temporal, 76.5 not; image-only denoise 113.5 and 114.4).
   // 1024^2: always (4 images, denoise 1131 against 1425 with every access cached and
   // rows not in strips).
-  static bool band_nt(const BandMap& map, int nimg, bool rows) {
+  static bool band_nt(const BandMap& map, int nimg, bool rows, int beside) {
     if (L == 512) return !(rows && nimg == 1);
-    return L >= 1024 || (L == 256 && map.nbands * (long long)nimg >= 480);
+    if (L == 256) return beside ? beside * (long long)nimg >= 960 : map.nbands * (long long)nimg >= 480;
+    return L >= 1024;
   }
   // Calls fn with band_nt's answer as a type; a size has the forms its rule can choose.
   template <class F>
@@ -1393,9 +1396,9 @@ struct Launch {
   template <int CT>
   static hipError_t cols_dec_ct(const float2* Y1, long long ys, float2* To, long long ts, const float2* Hm,
                                 const float2* Hb, const BandMap& map, int nimg, const float2* tw, hipStream_t s,
-                                bool pre, bool rows) {
+                                bool pre, bool rows, int beside) {
     const dim3 grid(L / 2 / CT, map.nbands, nimg), blk(ColCfg<L, CT>::T);
-    by_nt(band_nt(map, nimg, rows), [&](auto nt) {
+    by_nt(band_nt(map, nimg, rows, beside), [&](auto nt) {
       if (pre)
         hipLaunchKernelGGL((k_cols_dec<L, CT, true, nt.value>), grid, blk, 0, s, Y1, ys, To, ts, Hm, Hb, map, tw);
       else
@@ -1411,9 +1414,10 @@ struct Launch {
   }
   template <int CT>
   static hipError_t cols_rec_ct(const float2* U, long long us, float2* Q, long long qs, const float2* Hm,
-                                const float2* Hb, const BandMap& map, int nimg, const float2* tw, hipStream_t s) {
+                                const float2* Hb, const BandMap& map, int nimg, const float2* tw, hipStream_t s,
+                                int beside) {
     const dim3 grid(L / 2 / CT, map.ngroups, nimg), blk(ColCfg<L, CT>::T);
-    by_nt(band_nt(map, nimg, false), [&](auto nt) {
+    by_nt(band_nt(map, nimg, false, beside), [&](auto nt) {
       hipLaunchKernelGGL((k_cols_rec<L, CT, nt.value>), grid, blk, 0, s, U, us, Q, qs, Hm, Hb, map, tw);
     });
     return hipGetLastError();
@@ -1421,9 +1425,9 @@ struct Launch {
   template <int CT>
   static hipError_t cols_dec3_ct(const float2* Y1, long long ys, float2* To, long long ts, const float2* Hm,
                                  const float2* Hb, const BandMap& map, int nimg, const float2* tw, hipStream_t s,
-                                 bool rows) {
+                                 bool rows, int beside) {
     if constexpr ((L == 512 && CT >= 4) || L == 1024)
-      by_nt(band_nt(map, nimg, rows), [&](auto nt) {
+      by_nt(band_nt(map, nimg, rows, beside), [&](auto nt) {
         hipLaunchKernelGGL((k_cols_dec3<L, CT, nt.value>), dim3(L / 2 / CT, map.nbands, nimg), dim3(CT * 64), 0, s, Y1,
                            ys, To, ts, Hm, Hb, map, tw);
       });
@@ -1450,20 +1454,20 @@ struct Launch {
   static constexpr int kDefaultTile = ColTile<L>::narrow ? 4 : (ColTile<L>::dflt < 8 ? ColTile<L>::dflt : 8);
   static hipError_t cols_dec(const float2* Y1, long long ys, float2* To, long long ts, const float2* Hm,
                              const float2* Hb, const BandMap& map, int nimg, const float2* tw, hipStream_t s, int ct,
-                             bool pre, bool rows) {
+                             bool pre, bool rows, int beside) {
     if (ct < 0) {
       if ((L != 512 && L != 1024) || !pre) return hipErrorInvalidValue;
-      if (ct == -2 && L == 1024) return cols_dec3_ct<2>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, rows);
-      if (ct == -4) return cols_dec3_ct<4>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, rows);
-      if (ct == -8) return cols_dec3_ct<8>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, rows);
+      if (ct == -2 && L == 1024) return cols_dec3_ct<2>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, rows, beside);
+      if (ct == -4) return cols_dec3_ct<4>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, rows, beside);
+      if (ct == -8) return cols_dec3_ct<8>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, rows, beside);
       return hipErrorInvalidValue;
     }
     if (ct == 0) ct = kDefaultTile;
     if (ct == 4 && ColTile<L>::narrow)
-      return cols_dec_ct<(ColTile<L>::narrow ? 4 : 8)>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, pre, rows);
-    if (ct == 8) return cols_dec_ct<8>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, pre, rows);
+      return cols_dec_ct<(ColTile<L>::narrow ? 4 : 8)>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, pre, rows, beside);
+    if (ct == 8) return cols_dec_ct<8>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, pre, rows, beside);
     if (ct == 16 && ColTile<L>::wide)
-      return cols_dec_ct<(ColTile<L>::wide ? 16 : 8)>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, pre, rows);
+      return cols_dec_ct<(ColTile<L>::wide ? 16 : 8)>(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, pre, rows, beside);
     return hipErrorInvalidValue;
   }
   static hipError_t cols_fwd(float2* Y1, long long ys, int nplanes, int nimg, const float2* tw, hipStream_t s, int ct) {
@@ -1474,7 +1478,8 @@ struct Launch {
     return hipErrorInvalidValue;
   }
   static hipError_t cols_rec(const float2* U, long long us, float2* Q, long long qs, const float2* Hm,
-                             const float2* Hb, const BandMap& map, int nimg, const float2* tw, hipStream_t s, int ct) {
+                             const float2* Hb, const BandMap& map, int nimg, const float2* tw, hipStream_t s, int ct,
+                             int beside) {
     if (ct == 0) ct = L == 1024 ? (nimg == 1 ? -2 : -4) : (L == 512 ? -4 : kDefaultTile);
     if (ct < 0) {
       if (L != 512 && L != 1024) return hipErrorInvalidValue;
@@ -1483,9 +1488,9 @@ struct Launch {
       if (ct == -8) return cols_rec3_ct<8>(U, us, Q, qs, Hm, Hb, map, nimg, tw, s);
       return hipErrorInvalidValue;
     }
-    if (ct == 4 && ColTile<L>::narrow) return cols_rec_ct<(ColTile<L>::narrow ? 4 : 8)>(U, us, Q, qs, Hm, Hb, map, nimg, tw, s);
-    if (ct == 8) return cols_rec_ct<8>(U, us, Q, qs, Hm, Hb, map, nimg, tw, s);
-    if (ct == 16 && ColTile<L>::wide) return cols_rec_ct<(ColTile<L>::wide ? 16 : 8)>(U, us, Q, qs, Hm, Hb, map, nimg, tw, s);
+    if (ct == 4 && ColTile<L>::narrow) return cols_rec_ct<(ColTile<L>::narrow ? 4 : 8)>(U, us, Q, qs, Hm, Hb, map, nimg, tw, s, beside);
+    if (ct == 8) return cols_rec_ct<8>(U, us, Q, qs, Hm, Hb, map, nimg, tw, s, beside);
+    if (ct == 16 && ColTile<L>::wide) return cols_rec_ct<(ColTile<L>::wide ? 16 : 8)>(U, us, Q, qs, Hm, Hb, map, nimg, tw, s, beside);
     return hipErrorInvalidValue;
   }
 };
@@ -1525,8 +1530,8 @@ hipError_t launch_rows_c2r_mask_r2c(int L, const PlaneSet& Tin, const PlaneSet& 
 
 hipError_t launch_cols_dec(int L, const float2* Y1, long long ys, float2* To, long long ts, const float2* Hm,
                            const float2* Hb, const BandMap& map, int nimg, const float2* tw, hipStream_t s, int ct,
-                           bool pre, bool rows) {
-  SHX_BY_L(L, LT::cols_dec(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, ct, pre, rows))
+                           bool pre, bool rows, int beside) {
+  SHX_BY_L(L, LT::cols_dec(Y1, ys, To, ts, Hm, Hb, map, nimg, tw, s, ct, pre, rows, beside))
 }
 
 hipError_t launch_cols_fwd(int L, float2* Y1, long long ys, int nplanes, int nimg, const float2* tw, hipStream_t s,
@@ -2751,8 +2756,9 @@ bool col_tile_ok(int L, int ct) {
 }
 
 hipError_t launch_cols_rec(int L, const float2* U, long long us, float2* Q, long long qs, const float2* Hm,
-                           const float2* Hb, const BandMap& map, int nimg, const float2* tw, hipStream_t s, int ct) {
-  SHX_BY_L(L, LT::cols_rec(U, us, Q, qs, Hm, Hb, map, nimg, tw, s, ct))
+                           const float2* Hb, const BandMap& map, int nimg, const float2* tw, hipStream_t s, int ct,
+                           int beside) {
+  SHX_BY_L(L, LT::cols_rec(U, us, Q, qs, Hm, Hb, map, nimg, tw, s, ct, beside))
 }
 
 }  // namespace shx

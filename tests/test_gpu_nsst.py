@@ -283,6 +283,30 @@ def test_batch_equals_its_parts_across_the_store_rule(api, L, nimg, part, ct):
     shear.close()
 
 
+def test_side_by_side_scales_across_the_store_rule(api):
+    """A plan whose scales run side by side (level pyramid) stores its band
+    spectra non-temporally from 960 planes on: 20 images of 256^2 equal two
+    plans of 10, bit for bit."""
+    L, nimg, part = 256, 20, 10
+    print("case store rule, scales side by side", flush=True)
+    shear = api.make_dictionary(L)
+    assert 48 * part < 960 <= 48 * nimg
+    xg = to_gpu(np.stack([image(L, seed=90 + i)[1] for i in range(nimg)]))
+
+    def run(x):
+        b = api.Batch(shear, x.shape[0])
+        c, out = b.alloc_coeffs(), torch.empty_like(x)
+        b.denoise(x, c, torch.full((x.shape[0], shear.nbands), 40.0, device="cuda"), out)
+        torch.cuda.synchronize()
+        b.close()
+        return c, out
+    whole = run(xg)
+    for i in range(0, nimg, part):
+        for got, ref in zip(run(xg[i:i + part].contiguous()), whole):
+            assert torch.equal(got, ref[i:i + part])
+    shear.close()
+
+
 @pytest.mark.parametrize("parallel", [False, True])
 def test_mixed_size_batches_in_one_graph(api, parallel):
     print("case mixed graph parallel=%s" % parallel, flush=True)
