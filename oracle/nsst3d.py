@@ -1,6 +1,6 @@
 """FP64 CPU oracle for the 3D shearlet volume transform.
 
-TEST INFRASTRUCTURE ONLY.  This module is the checker that the HIP library is
+TEST INFRASTRUCTURE ONLY.  This module is the oracle that the HIP library is
 compared against.  Only ``tests/``, ``__graft_entry__.smoke()`` and the
 ``cpu_baseline`` leg of ``bench.py`` may import it; the product path
 (``shearcuda_amd``) never does.
